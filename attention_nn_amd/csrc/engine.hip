@@ -1050,6 +1050,7 @@ int ann_decode_step(ann_ctx* c, const int32_t* tokens, int32_t B, const ann_samp
   const bool greedy = s->temperature == 0.f;
   // set up before the step may be captured into a graph below
   if (cand_route(c, B, greedy)) HIPCHK(sample_prepare());
+  HIPCHK(gemm_ring_prepare());
   rc = clear_decode_state(c, st);   // tags, tickets, partials and the error word
   if (rc) return rc;
   // The batch-1 persistent step is one kernel (plus the sampler when not

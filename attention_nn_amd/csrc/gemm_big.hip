@@ -1,10 +1,9 @@
-// Large projections y = a @ W^T (W stored (N, K) bf16) of the prefill and the
-// training forward: 256 x 256 (or 256 x 192) output tiles of four waves of
-// 128 x 128 (128 x 96), one work-group (one wave per SIMD) per CU,
-// v_mfma_f32_16x16x32_bf16.  The projection routing sends the fc (relu^2),
-// o-proj (attention residual) and proj (MLP residual) projections here (see
-// gemm_big_routes for the measurements); it serves the plain and QKV
-// epilogues as well when called directly.
+// The MLP's output projection x = r1 x + p1 (h @ W^T) (W stored (N, K) bf16)
+// where h is larger than the memory-side cache (gemm_big_routes has the
+// measurements against k_gemm_ring): 256 x 256 (or 256 x 192) output tiles of
+// four waves of 128 x 128 (128 x 96), one work-group (one wave per SIMD) per
+// CU, v_mfma_f32_16x16x32_bf16 -- the tile that moves the fewest bytes per
+// flop.
 //
 // Main loop (K tiles of 64, two LDS stages, one barrier per K tile):
 //   * the 256 accumulators of a wave live in AGPRs: the MFMA is issued as
@@ -28,26 +27,16 @@
 //     c ^ ((r >> 1) & 7): conflict-free for the chunk stores and the
 //     16-row fragment reads.
 // The MFMA operands are swapped (C^T = W A^T) so that a lane holds four
-// consecutive columns of one row.  Epilogue: the tile is rounded to bf16 (every
-// epilogue here starts from bf16(y), as the reference's eager ops do; relu^2
-// is applied at this point) into LDS (row pitch 264: the 8-byte writes of 16
-// rows spread over the banks), then each thread handles 16-byte row chunks:
-// plain / relu^2 copies, the residual mixes (x, x0 read and x written as
-// 16-byte words, the first batch loaded before the staging), or the QKV
-// epilogue of each 128-column half (QK-norm, RoPE, q and KV-cache writes).
-// With one wave per SIMD nothing hides the epilogue's VALU work, so every
-// eager rounding is a packed pair conversion (v_cvt_pk_bf16_f32): per-work-
-// group stamps of the 64 x 512-token prefill put the fc epilogue at 5.7-7.5
-// us per tile after this, 7.3 before (main loop ~21 us).  Work-group i
-// runs on XCD i % 8; each XCD takes a contiguous range of tiles, N-fastest, so
-// the N tiles of an M block share its A rows in that XCD's L2.
-// Measured against the four prefill shapes (M = 32768) with a plain store:
-// 0.81 / 0.70 / 0.96 / 1.04 PFLOP/s for N x K = 2304 x 768, 768 x 768,
-// 3072 x 768, 768 x 3072 (hipBLASLt: 0.87 / 0.83 / 1.17 / 1.29).
-#include <stdlib.h>
+// consecutive columns of one row.  Epilogue: the tile is rounded to bf16 (as
+// the reference's eager ops do) into LDS (row pitch 264: the 8-byte writes of
+// 16 rows spread over the banks), then each thread mixes 16-byte row chunks (x
+// read and written as 16-byte words, the first batch loaded before the
+// staging).  With one wave per SIMD nothing hides the epilogue's VALU work, so
+// every eager rounding is a packed pair conversion (v_cvt_pk_bf16_f32).
+// Work-group i runs on XCD i % 8; each XCD takes a contiguous range of tiles,
+// N-fastest, so the N tiles of an M block share its A rows in that XCD's L2.
 #include <type_traits>
 #include "common.h"
-#include "epilogue.h"
 #include "launch.h"
 
 namespace ann {
@@ -56,9 +45,7 @@ namespace {
 
 constexpr int BG_BM = 256, BG_BN = 256, BG_BK = 64;   // BG_BN: the widest tile
 constexpr int BG_EP = 264;   // bf16 row pitch of the staged output tile
-#ifndef BG_EB
-#define BG_EB 8              // residual epilogue: 16-byte chunks per thread loaded at once
-#endif
+constexpr int BG_EB = 8;     // residual epilogue: 16-byte chunks per thread loaded at once
 constexpr size_t BG_LDS_MAIN = (size_t)2 * (BG_BM + BG_BN) * BG_BK * 2;
 constexpr size_t BG_LDS_EPI = (size_t)BG_BM * BG_EP * 2;
 constexpr size_t BG_LDS = BG_LDS_MAIN > BG_LDS_EPI ? BG_LDS_MAIN : BG_LDS_EPI;
@@ -97,11 +84,10 @@ __device__ __forceinline__ void bg_wait_lgkm() {
 }  // namespace
 
 
-template <int EPI, int BN>
+template <int BN>
 __global__ __launch_bounds__(256, 1) void k_gemm_big(const bf16_t* A, int lda, const bf16_t* W,
                                                      int M, int N, int K, EpiArgs ea) {
   static_assert(BN == 256 || BN == 192, "tile width");
-  static_assert(EPI != EPI_QKV || BN == 256, "the QKV epilogue takes 128-column head halves");
   constexpr int NJ = BN / 32;    // 16-column blocks of a wave (two waves across the tile)
   constexpr int NWU = BN / 32;   // W chunks per thread and K tile
   constexpr int CPR = BN / 8;    // 16-byte chunks per output row
@@ -218,24 +204,20 @@ __global__ __launch_bounds__(256, 1) void k_gemm_big(const bf16_t* A, int lda, c
     __syncthreads();
   }
 
-  // residual epilogues: x (and x0) chunks of the first batch loaded before the
-  // staging (chunk q = tid + 256 u is row q / CPR, columns 8 (q % CPR); rows
-  // past M read row M - 1 and are never stored)
-  constexpr bool RES = EPI == EPI_RESID_ATTN || EPI == EPI_RESID_MLP;
-  static_assert(!RES || CPR % BG_EB == 0, "whole batches");
-  bg_u32x4 xv[2][BG_EB], zv[2][BG_EB];
+  // residual epilogue: x chunks of the first batch loaded before the staging
+  // (chunk q = tid + 256 u is row q / CPR, columns 8 (q % CPR); rows past M
+  // read row M - 1 and are never stored)
+  static_assert(CPR % BG_EB == 0, "whole batches");
+  bg_u32x4 xv[2][BG_EB];
   auto res_load = [&](int b) {
 #pragma unroll
     for (int e = 0; e < BG_EB; ++e) {
       const int q = tid + 256 * (b * BG_EB + e);
       const size_t i = (size_t)min(m0 + q / CPR, M - 1) * ea.ldr + n0 + (q % CPR) * 8;
       xv[b & 1][e] = *(const bg_u32x4*)(ea.x + i);
-      if constexpr (EPI == EPI_RESID_ATTN) zv[b & 1][e] = *(const bg_u32x4*)(ea.x0 + i);
     }
   };
-  if constexpr (RES) res_load(0);
-  QkvRows<BG_BM> pr;
-  if constexpr (EPI == EPI_QKV) qkv_prefetch<BG_BM>(ea, m0, M, tid, pr);
+  res_load(0);
   // ---- stage bf16(y): lane holds row m = block row + r16, columns 4 kg ..
   bf16_t* st = smem;
 #pragma unroll
@@ -244,188 +226,87 @@ __global__ __launch_bounds__(256, 1) void k_gemm_big(const bf16_t* A, int lda, c
     for (int j = 0; j < NJ; ++j) {
       const int ml = wm * 128 + i * 16 + r16, nl = wn * (BN / 2) + j * 16 + 4 * kg;
       const bg_floatx4 v = acc[i][j];
-      uint2 w;
-      if constexpr (EPI == EPI_RELU2)   // relu^2 applied here: the copy below only moves bytes
-        w = make_uint2(relu2_pair(v[0], v[1]), relu2_pair(v[2], v[3]));
-      else
-        w = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
-      *(uint2*)(st + ml * BG_EP + nl) = w;
+      *(uint2*)(st + ml * BG_EP + nl) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
     }
   __syncthreads();
-
-  if constexpr (EPI == EPI_QKV) {
-    qkv_tile_epilogue<BG_BM, BG_EP>(ea, st, m0, n0, M, tid, pr);
-    qkv_tile_epilogue<BG_BM, BG_EP>(ea, st + 128, m0, n0 + 128, M, tid, pr);
-    return;
-  } else {
-    // 16-byte row chunks: chunk q = tid + 256 u is row q / CPR, columns 8 (q % CPR)
-    if constexpr (RES) {
-      // batch b + 1's loads fly while batch b is mixed and stored
-      float lam[5];
+  // 16-byte row chunks; batch b + 1's loads fly while batch b is mixed and stored
+  float lam[5];
 #pragma unroll
-      for (int e = 0; e < 5; ++e) lam[e] = ea.lam[e];
+  for (int e = 0; e < 5; ++e) lam[e] = ea.lam[e];
 #pragma unroll
-      for (int b = 0; b < CPR / BG_EB; ++b) {
-        if (b + 1 < CPR / BG_EB) res_load(b + 1);
+  for (int b = 0; b < CPR / BG_EB; ++b) {
+    if (b + 1 < CPR / BG_EB) res_load(b + 1);
 #pragma unroll
-        for (int e = 0; e < BG_EB; ++e) {
-          const int q = tid + 256 * (b * BG_EB + e);
-          const int ml = q / CPR, c8 = (q % CPR) * 8;
-          const bg_u32x4 y = *(const bg_u32x4*)(st + ml * BG_EP + c8);
-          const bg_u32x4 x = xv[b & 1][e];
-          bg_u32x4 o;
+    for (int e = 0; e < BG_EB; ++e) {
+      const int q = tid + 256 * (b * BG_EB + e);
+      const int ml = q / CPR, c8 = (q % CPR) * 8;
+      const bg_u32x4 y = *(const bg_u32x4*)(st + ml * BG_EP + c8);
+      const bg_u32x4 x = xv[b & 1][e];
+      bg_u32x4 o;
 #pragma unroll
-          for (int f = 0; f < 4; ++f) {
-            if constexpr (EPI == EPI_RESID_ATTN) o[f] = mix_attn_pair(lam, x[f], zv[b & 1][e][f], y[f]);
-            else o[f] = mix_mlp_pair(lam, x[f], y[f]);
-          }
-          if (m0 + ml < M) *(bg_u32x4*)(ea.x + (size_t)(m0 + ml) * ea.ldr + n0 + c8) = o;
-        }
-      }
-      return;
-    }
-    // plain / relu^2 (already applied): 16-byte row chunks, eight LDS reads
-    // in flight per thread; the fc output goes out with non-temporal stores
-    // (it is read back only by the next projection; 10 us less per fc call)
-    static_assert(CPR % 8 == 0, "whole batches");
-#pragma unroll
-    for (int u0 = 0; u0 < CPR; u0 += 8) {
-      bg_u32x4 w[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int q = tid + 256 * (u0 + e);
-        w[e] = *(const bg_u32x4*)(st + (q / CPR) * BG_EP + (q % CPR) * 8);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int q = tid + 256 * (u0 + e);
-        const int m = m0 + q / CPR, n = n0 + (q % CPR) * 8;
-        if (m < M) {
-          bg_u32x4* dst = (bg_u32x4*)(ea.out + (size_t)m * ea.ldo + n);
-          if constexpr (EPI == EPI_RELU2) __builtin_nontemporal_store(w[e], dst);
-          else *dst = w[e];
-        }
-      }
+      for (int f = 0; f < 4; ++f) o[f] = mix_mlp_pair(lam, x[f], y[f]);
+      if (m0 + ml < M) *(bg_u32x4*)(ea.x + (size_t)(m0 + ml) * ea.ldr + n0 + c8) = o;
     }
   }
 }
 
-static int big_cus() {
-  static int cus = 0;
-  if (!cus) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-  }
+int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus <= 0)
+    return 256;
   return cus;
 }
 
-// Whether the projection routing (gemm()) sends (epi, M, N) here.  In the
-// 64 x 512-token prefill, per layer against the two-work-groups-per-CU tiles
-// of k_gemm_2w (rocprof, one box): fc (relu^2) 185 us here; o-proj (attention
-// residual) 79 us here with 192-column tiles (103 with 256, 108 in k_gemm_2w);
-// proj (MLP residual) 159 us here with 192-column tiles against 199 in
-// k_gemm_2w.  QKV: 165 us here against 150 in k_gemm_2w at 64 x 512 tokens,
-// whose 1152 tiles leave the fifth round of 256 CUs half empty; with whole
-// rounds it wins (16 x 7680 tokens: 4320 tiles, 565 -> 535 us; d 1536 at
-// 128 x 1024: 9216 tiles, 2072 -> 1816 us), so QKV comes here when the last
-// round's idle CUs are under 5% of all rounds.  The kernel still serves every
-// epilogue of gemm_big() when called directly.
-bool gemm_big_routes(int epi, int M, int N) {
-  if (epi == EPI_RELU2 || epi == EPI_RESID_ATTN || epi == EPI_RESID_MLP) return true;
-  if (epi != EPI_QKV || N % BG_BN) return false;
-  const long long cus = big_cus(), tiles = (long long)((M + BG_BM - 1) / BG_BM) * (N / BG_BN);
-  const long long slots = (tiles + cus - 1) / cus * cus;
-  return (slots - tiles) * 20 < slots;
-}
+// Whether an (M, N) = (rows, d) product over K comes here instead of
+// k_gemm_ring: where A is 384 MB or more, past the memory-side cache.  Ring
+// against here, in us: d 768 (K 3072) at 32768 rows 137 / 150, at 65536 300 /
+// 284, at 122880 557 / 536; d 1536 (K 6144) at 16384 rows 272 / 276, at 32768
+// 550 / 509, at 65536 1076 / 989, at 131072 2136 / 1975.
+bool gemm_big_routes(int M, int K) { return (long long)M * K >= 192LL << 20; }
 
 // Tile width for an M x N output: 256 or 192 columns, whichever needs fewer
 // CU-rounds times columns (one work-group per CU), a 192-column tile counted
-// 15% dearer per column (less reuse of each A tile: the cfg4 fc shape, 480 x 16
-// tiles of 192 against 480 x 12 of 256, measured 818 against 713 us).  N = 768
-// at M = 32768: 384 tiles of 256 fill 1.5 rounds of 256 CUs, 512 tiles of 192
-// two whole rounds (o-proj 79 against 103 us).  The QKV epilogue needs 256
-// (head halves).
-// ANN_GEMM_BIG_BN=256 / 192 forces one where it divides N (read once per
-// process).
-static int big_bn(int epi, int M, int N) {
-  static int force = -1;
-  if (force < 0) {
-    const char* e = getenv("ANN_GEMM_BIG_BN");
-    force = e ? atoi(e) : 0;
-  }
-  const int cus = big_cus();
-  const bool ok192 = epi != EPI_QKV && N % 192 == 0, ok256 = N % 256 == 0;
-  if (!ok192) return 256;
-  if (!ok256) return 192;
-  if (force == 192 || force == 256) return force;
+// 15% dearer per column (less reuse of each A tile: 480 x 16 tiles of 192
+// against 480 x 12 of 256 measured 818 against 713 us).
+static int big_bn(int M, int N) {
+  static const int cus = device_cus();
+  if (N % 192) return 256;
+  if (N % 256) return 192;
   const long long ntm = (M + BG_BM - 1) / BG_BM;
   auto rounds = [&](int bn) { return (ntm * (N / bn) + cus - 1) / cus; };
   return rounds(192) * 192 * 115 < rounds(256) * 256 * 100 ? 192 : 256;
 }
 
-// Whether gemm_big can take (epi, M, N, K): whole 256- or 192-column tiles,
-// 64-deep K tiles, 16-byte aligned rows and outputs, and enough tiles (at
-// least 96) for the one-work-group-per-CU kernel to fill the chip.
-bool gemm_big_fits(int epi, const bf16_t* A, int lda, int M, int N, int K, const EpiArgs& ea) {
+// Whether gemm_big can take (M, N, K): whole 256- or 192-column tiles, 64-deep
+// K tiles, 16-byte aligned rows, and enough tiles (at least 96) for the one-
+// work-group-per-CU kernel to fill the chip.
+bool gemm_big_fits(const bf16_t* A, int lda, int M, int N, int K, const EpiArgs& ea) {
   if (M < 512 || N % 64 || K % BG_BK || K < BG_BK || lda % 8 || ((uintptr_t)A & 15)) return false;
-  const int bn = big_bn(epi, M, N);
+  const int bn = big_bn(M, N);
   if (N % bn) return false;
   if ((long long)((M + BG_BM - 1) / BG_BM) * (N / bn) < 96) return false;
-  switch (epi) {
-    case EPI_STORE:
-    case EPI_RELU2:
-      return ea.out && ea.ldo % 8 == 0 && ((uintptr_t)ea.out & 15) == 0;
-    case EPI_RESID_ATTN:
-      return ea.x && ea.x0 && ea.lam && ea.ldr % 8 == 0 &&
-             (((uintptr_t)ea.x | (uintptr_t)ea.x0) & 15) == 0;
-    case EPI_RESID_MLP:
-      return ea.x && ea.lam && ea.ldr % 8 == 0 && ((uintptr_t)ea.x & 15) == 0;
-    case EPI_QKV:
-      return true;   // gemm_qkv_fits has been checked by the caller
-    default:
-      return false;
-  }
+  return ea.x && ea.lam && ea.ldr % 8 == 0 && ((uintptr_t)ea.x & 15) == 0;
 }
 
-template <int EPI, int BN>
+template <int BN>
 static hipError_t launch_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                              const EpiArgs& ea, hipStream_t st) {
-  static bool attr = false;
-  if (!attr) {
-    const hipError_t e = hipFuncSetAttribute((const void*)k_gemm_big<EPI, BN>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)BG_LDS);
-    if (e != hipSuccess) return e;
-    attr = true;
-  }
+  static const hipError_t attr = hipFuncSetAttribute(
+      (const void*)k_gemm_big<BN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BG_LDS);
+  if (attr != hipSuccess) return attr;
   const int nt = ((M + BG_BM - 1) / BG_BM) * (N / BN);
   const int grid = (nt + 7) / 8 * 8;
-  hipLaunchKernelGGL((k_gemm_big<EPI, BN>), dim3(grid), dim3(256), BG_LDS, st, A, lda, W, M, N, K,
-                     ea);
+  hipLaunchKernelGGL((k_gemm_big<BN>), dim3(grid), dim3(256), BG_LDS, st, A, lda, W, M, N, K, ea);
   return hipGetLastError();
 }
 
-hipError_t gemm_big(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+hipError_t gemm_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                     const EpiArgs& ea, hipStream_t st) {
-  if (!gemm_big_fits(epi, A, lda, M, N, K, ea)) return hipErrorInvalidValue;
-  const bool w192 = big_bn(epi, M, N) == 192;
-  switch (epi) {
-#define ANN_BIG_CASE(E)                                                              \
-  case E:                                                                            \
-    return w192 ? launch_big<E, 192>(A, lda, W, M, N, K, ea, st)                     \
-                : launch_big<E, 256>(A, lda, W, M, N, K, ea, st);
-    ANN_BIG_CASE(EPI_STORE)
-    ANN_BIG_CASE(EPI_RELU2)
-    ANN_BIG_CASE(EPI_RESID_ATTN)
-    ANN_BIG_CASE(EPI_RESID_MLP)
-#undef ANN_BIG_CASE
-    case EPI_QKV: return launch_big<EPI_QKV, 256>(A, lda, W, M, N, K, ea, st);
-    default: return hipErrorInvalidValue;
-  }
+  if (!gemm_big_fits(A, lda, M, N, K, ea)) return hipErrorInvalidValue;
+  return big_bn(M, N) == 192 ? launch_big<192>(A, lda, W, M, N, K, ea, st)
+                             : launch_big<256>(A, lda, W, M, N, K, ea, st);
 }
 
 }  // namespace ann
-

@@ -1,0 +1,400 @@
+// Projections y = a @ W^T (W stored (N, K) bf16) of more than 128 rows: one
+// ordinary prompt, a batch's prompts, the scoring of a text, the training
+// forward.  K tiles of 64 are streamed straight into a ring of NS LDS stages
+// (global_load_lds_dwordx4, no register staging), one barrier per K tile; the
+// output tile is chosen by the shape (ring_pick).
+//
+// What bounds it.  A lone work-group and a full CU take the same time per K
+// tile of a 64 x 64 or 128 x 64 tile, 0.2 and 0.31 us: 16 and 24 KB through the
+// CU's load path, about 80 GB/s per CU (38 of its 64 bytes per clock).  So a
+// shape that leaves CUs idle wants small tiles on all of them, and a shape
+// that fills them wants large tiles, which move fewer bytes per flop: 128 x
+// 128 takes 0.51 us and 128 x 192 0.64 us per K tile, where the MFMAs alone
+// take 0.31 and 0.46 (1.75 PFLOP/s, the form's measured ceiling).  Two
+// work-groups share a CU at every tile: their barriers fall apart in time, so
+// one reads LDS and waits while the other multiplies, and one's epilogue runs
+// under the other's main loop.  One work-group of eight waves with the same
+// tiles (256 x 128, two or three stages) is slower for that reason (proj of
+// 32768 rows, d 768: 160 against 147 us), as are K tiles of 32 (half cache
+// lines: 171) and v_mfma_f32_32x32x16 (164 against 133 at 128 x 128).
+#include <type_traits>
+#include "common.h"
+#include "epilogue.h"
+#include "launch.h"
+
+namespace ann {
+
+namespace {
+
+constexpr int RG_BK = 64;
+constexpr int RG_RB = RG_BK * 2;   // bytes of an LDS row
+
+typedef __bf16 rg_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float rg_floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t rg_u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void rg_lds_void;
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void rg_static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    rg_static_for<I + 1, N>(f);
+  }
+}
+
+// This wave's loads but the newest N have landed and its LDS reads are done
+// (another wave's load may overwrite what they read), then every wave's.
+template <int N>
+__device__ __forceinline__ void rg_wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+}
+
+template <int BM, int BN, int NS>
+constexpr size_t rg_lds_bytes() {
+  const size_t ring = (size_t)NS * (BM + BN) * RG_RB, epi = (size_t)BM * (BN + 8) * 2;
+  return ring > epi ? ring : epi;
+}
+
+}  // namespace
+
+// WR x WC waves.  gm: tile rows per group of the tile order.
+template <int EPI, int BM, int BN, int NS, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_ring(
+    const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int M, int N, int K,
+    int gm, EpiArgs ea) {
+  constexpr int NW = WR * WC, TH = 64 * NW;
+  constexpr int WM = BM / WR, MT = WM / 16;
+  constexpr int WN = BN / WC, NT = WN / 16;
+  constexpr int LA = BM / 8 / NW, LW = BN / 8 / NW;   // 1 KB loads per wave per K tile
+  constexpr int SB = (BM + BN) * RG_RB;               // bytes of a stage
+  constexpr int CPR = BN / 8, NCH = BM * CPR / TH, CP = BN + 8;
+  constexpr bool RES = EPI == EPI_RESID_ATTN || EPI == EPI_RESID_MLP;
+  // the residual operands: loaded first where the tile is small (a few
+  // registers, and nothing else hides the latency), after the main loop else
+  constexpr bool EARLY = RES && BM * BN <= 128 * 64;
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && BM * CPR % TH == 0, "whole loads");
+  static_assert(EPI != EPI_QKV || (BN == 128 && TH == 256), "whole heads per tile");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rg_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wv / WC, wn = wv % WC;
+  // Tile order: each XCD (work-group b runs on XCD b % 8) takes a contiguous
+  // range of the tiles, which are ordered in groups of gm tile rows, column
+  // by column, so that the tiles at work together on an XCD share A and W
+  // rows in its L2 (a bijection of the grid, correct under any dispatch).
+  // gm 4 against row by row, 128 x 128 tiles: qkv of 8192 rows, d 1536, 134 ->
+  // 120 us, fc 167 -> 142; d 768 up to 10%; gm 8 equal, 16 slower.
+  int tm, tn;
+  {
+    const int nbn = gridDim.x, nbm = gridDim.y, total = nbn * nbm;
+    const int bid = blockIdx.y * nbn + blockIdx.x;
+    const int x = bid & 7, q = total >> 3, r = total & 7;
+    const int t = x * q + min(x, r) + (bid >> 3);
+    const int g = t / (gm * nbn), rem = t - g * gm * nbn;
+    const int h = min(gm, nbm - g * gm);
+    tn = rem / h;
+    tm = g * gm + rem - tn * h;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int KT = K / RG_BK;
+
+  // chunk q = tid + TH u of the output tile: row q / CPR, columns 8 (q % CPR)
+  uint4 xv[RES ? NCH : 1], zv[EPI == EPI_RESID_ATTN ? NCH : 1];
+  auto res_load = [&]() {
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int q = tid + TH * u;
+      const size_t i = (size_t)min(m0 + q / CPR, M - 1) * ea.ldr + min(n0 + (q % CPR) * 8, N - 8);
+      xv[u] = *(const uint4*)(ea.x + i);
+      if constexpr (EPI == EPI_RESID_ATTN) zv[u] = *(const uint4*)(ea.x0 + i);
+    }
+  };
+  if constexpr (EARLY) res_load();
+
+  // load u of this wave fills rows 8 (NW u + wv) .. + 7 of the operand's tile
+  // in LDS: lane l row l >> 3, slot l & 7, which holds logical 16-byte chunk
+  // (l & 7) ^ ((row >> 1) & 7) -- conflict-free for the 16-row fragment reads.
+  // Rows past M / N repeat the last one (they feed outputs never stored).
+  const bf16_t* pa[LA];
+  const bf16_t* pw[LW];
+#pragma unroll
+  for (int u = 0; u < LA; ++u) {
+    const int r = 8 * (NW * u + wv) + (lane >> 3);
+    pa[u] = A + (size_t)min(m0 + r, M - 1) * lda + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+  }
+#pragma unroll
+  for (int u = 0; u < LW; ++u) {
+    const int r = 8 * (NW * u + wv) + (lane >> 3);
+    pw[u] = W + (size_t)min(n0 + r, N - 1) * K + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+  }
+  // (the builtin's operands have plain types: clang's host pass drops a kernel
+  // in which a type-dependent call of its 16-byte form is instantiated)
+  auto issue = [&](int kt, int s) {
+    unsigned char* st = rg_smem + s * SB;
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const bf16_t* src = pa[u] + kt * RG_BK;
+      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
+    }
+    st += BM * RG_RB;
+#pragma unroll
+    for (int u = 0; u < LW; ++u) {
+      const bf16_t* src = pw[u] + kt * RG_BK;
+      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
+    }
+  };
+
+  rg_floatx4 acc[NT][MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[j][i] = (rg_floatx4){0.f, 0.f, 0.f, 0.f};
+
+  // block (N block j, M block i) of C^T = W A^T: a lane holds four consecutive
+  // columns of one row.  The k steps of 32 run in order, as in every GEMM
+  // here: the same bits whatever the tile.
+  const int r16 = lane & 15, kg = lane >> 4, sw = (r16 >> 1) & 7;
+  const int oa = (wm * WM + r16) * RG_RB, ow = BM * RG_RB + (wn * WN + r16) * RG_RB;
+  const int c0 = (kg ^ sw) << 4, c1 = ((4 + kg) ^ sw) << 4;
+  auto compute = [&](int s) {
+    const unsigned char* st = rg_smem + s * SB;
+    rg_bf16x8 a[2][MT], w[2][NT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        w[h][j] = *(const rg_bf16x8*)(st + ow + j * 16 * RG_RB + (h ? c1 : c0));
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        a[h][i] = *(const rg_bf16x8*)(st + oa + i * 16 * RG_RB + (h ? c1 : c0));
+    }
+    __builtin_amdgcn_sched_barrier(0);   // all reads in flight, then the MFMAs
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h][j], a[h][i], acc[j][i], 0, 0, 0);
+  };
+
+  // ring: K tile t in stage t % NS, loaded NS - 1 tiles ahead.  The barrier
+  // that follows the wait for tile t also says that every wave is done with
+  // the stage of tile t - 1, which tile t + NS - 1 then overwrites.  (With
+  // fewer K tiles than that the last one is loaded again, and not used.)
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t) issue(min(t, KT - 1), t);
+  int s = 0;
+  for (int t = 0; t < KT - (NS - 1); ++t) {
+    rg_wait_barrier<(NS - 2) * (LA + LW)>();
+    issue(t + NS - 1, s == 0 ? NS - 1 : s - 1);
+    compute(s);
+    s = s + 1 == NS ? 0 : s + 1;
+  }
+  rg_static_for<0, NS - 1>([&](auto tc) __attribute__((always_inline)) {
+    rg_wait_barrier<(NS - 2 - decltype(tc)::value) * (LA + LW)>();
+    if (decltype(tc)::value < KT) compute(s);
+    s = s + 1 == NS ? 0 : s + 1;
+  });
+
+  // epilogue: bf16(y) staged in LDS, then 16-byte row chunks
+  if constexpr (RES && !EARLY) res_load();
+  QkvRows<BM> pr;
+  if constexpr (EPI == EPI_QKV) qkv_prefetch<BM>(ea, m0, M, tid, pr);
+  __syncthreads();   // every wave is done with the last K tile
+  bf16_t* tile = (bf16_t*)rg_smem;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const rg_floatx4 y = acc[j][i];
+      uint2 v;
+      if constexpr (EPI == EPI_RELU2) v = make_uint2(relu2_pair(y[0], y[1]), relu2_pair(y[2], y[3]));
+      else v = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
+      *(uint2*)(tile + (wm * WM + i * 16 + r16) * CP + wn * WN + j * 16 + 4 * kg) = v;
+    }
+  __syncthreads();
+  if constexpr (EPI == EPI_QKV) {
+    qkv_tile_epilogue<BM, CP>(ea, tile, m0, n0, M, tid, pr);
+  } else {
+    float lam[5];
+    if constexpr (RES) {
+#pragma unroll
+      for (int e = 0; e < 5; ++e) lam[e] = ea.lam[e];
+    }
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int q = tid + TH * u, ml = q / CPR, c8 = (q % CPR) * 8;
+      const int m = m0 + ml, n = n0 + c8;
+      const uint4 y = *(const uint4*)(tile + ml * CP + c8);
+      if (m >= M || n >= N) continue;
+      if constexpr (RES) {
+        uint4 o;
+        if constexpr (EPI == EPI_RESID_ATTN) {
+          o.x = mix_attn_pair(lam, xv[u].x, zv[u].x, y.x);
+          o.y = mix_attn_pair(lam, xv[u].y, zv[u].y, y.y);
+          o.z = mix_attn_pair(lam, xv[u].z, zv[u].z, y.z);
+          o.w = mix_attn_pair(lam, xv[u].w, zv[u].w, y.w);
+        } else {
+          o.x = mix_mlp_pair(lam, xv[u].x, y.x);
+          o.y = mix_mlp_pair(lam, xv[u].y, y.y);
+          o.z = mix_mlp_pair(lam, xv[u].z, y.z);
+          o.w = mix_mlp_pair(lam, xv[u].w, y.w);
+        }
+        *(uint4*)(ea.x + (size_t)m * ea.ldr + n) = o;
+      } else if constexpr (EPI == EPI_LOGITS) {
+        const size_t i = (size_t)m * ea.ldz + n;
+        if (ea.z) *(uint4*)(ea.z + i) = y;
+        if (ea.logits) {
+          *(float4*)(ea.logits + i) = make_float4(softcap(lo_f(y.x)), softcap(hi_f(y.x)),
+                                                  softcap(lo_f(y.y)), softcap(hi_f(y.y)));
+          *(float4*)(ea.logits + i + 4) = make_float4(softcap(lo_f(y.z)), softcap(hi_f(y.z)),
+                                                      softcap(lo_f(y.w)), softcap(hi_f(y.w)));
+        }
+      } else if constexpr (EPI == EPI_RELU2 && BN == 192) {
+        // a large fc output, read back once by the next projection: past the
+        // caches (fc of 32768 rows, d 768: 163 -> 157 us at 128 x 128)
+        __builtin_nontemporal_store(__builtin_bit_cast(rg_u32x4, y),
+                                    (rg_u32x4*)(ea.out + (size_t)m * ea.ldo + n));
+      } else {
+        *(uint4*)(ea.out + (size_t)m * ea.ldo + n) = y;
+      }
+    }
+  }
+}
+
+namespace {
+
+template <int EPI, int BM, int BN, int NS, int WR, int WC>
+hipError_t launch_ring(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                       const EpiArgs& ea, hipStream_t st) {
+  if (N % BN) return hipErrorInvalidValue;
+  const dim3 grid(N / BN, (M + BM - 1) / BM);
+  hipLaunchKernelGGL((k_gemm_ring<EPI, BM, BN, NS, WR, WC>), grid, dim3(64 * WR * WC),
+                     (rg_lds_bytes<BM, BN, NS>()), st, A, lda, W, M, N, K, 4, ea);
+  return hipGetLastError();
+}
+
+// dynamic LDS beyond 64 KB has to be asked for
+template <int EPI, int BM, int BN, int NS, int WR, int WC>
+bool ring_attr() {
+  return hipFuncSetAttribute((const void*)k_gemm_ring<EPI, BM, BN, NS, WR, WC>,
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)rg_lds_bytes<BM, BN, NS>()) == hipSuccess;
+}
+template <int EPI>
+bool ring_attrs() {
+  return ring_attr<EPI, 32, 64, 6, 1, 4>() && ring_attr<EPI, 64, 64, 4, 2, 2>() &&
+         ring_attr<EPI, 128, 64, 3, 2, 2>() && ring_attr<EPI, 128, 128, 2, 2, 2>() &&
+         ring_attr<EPI, 128, 192, 2, 2, 2>();
+}
+
+// The tiles, with the time per K tile of a work-group alone on its CU and of
+// one of two that share it, and what a launch takes besides, in ns (measured
+// on the o / proj / fc shapes of d 512, 768 and 1536).
+struct RingTile {
+  int bm, bn;
+  int alone, shared, fixed;
+};
+constexpr RingTile RING_TILES[] = {
+    {32, 64, 150, 145, 2800},   {64, 64, 207, 195, 2900},   {128, 64, 340, 290, 3600},
+    {128, 128, 590, 470, 4600}, {128, 192, 780, 660, 5000},
+    // QKV only (a 128-column tile holds whole heads)
+    {64, 128, 340, 290, 3600},  {192, 128, 780, 660, 5000}};
+constexpr int RING_N = 5, RING_QKV_N = 7;
+
+}  // namespace
+
+// The tile that is done first: the CU with the most work-groups takes them in
+// pairs (two are resident).  Measured against every tile at 130 .. 32768 rows
+// of d 512, 768 and 1536: within 5% of the best one at most shapes, 15% at
+// the worst.  One always fits (N is a multiple of 64, of 128 for QKV).
+static int ring_pick(int epi, int M, int N, int K) {
+  static const int cus = device_cus();
+  int best = -1;
+  long long best_ns = 0;
+  for (int i = 0; i < RING_QKV_N; ++i) {
+    const RingTile& t = RING_TILES[i];
+    if (epi == EPI_QKV ? t.bn != 128 : i >= RING_N) continue;
+    if (N % t.bn) continue;
+    const long long wgs = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn);
+    const long long n = (wgs + cus - 1) / cus;
+    const long long ns = K / RG_BK * (n / 2 * 2 * t.shared + n % 2 * t.alone) + t.fixed;
+    if (best < 0 || ns < best_ns) {
+      best = i;
+      best_ns = ns;
+    }
+  }
+  return best;
+}
+
+// Rows of A and of the epilogue's operands in 16-byte words, whole 64-column
+// tiles.
+bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                    const EpiArgs& ea) {
+  if (M < 1 || N < 64 || N % 64 || K < RG_BK || K % RG_BK || lda % 8 ||
+      (((uintptr_t)A | (uintptr_t)W) & 15))
+    return false;
+  switch (epi) {
+    case EPI_STORE:
+    case EPI_RELU2:
+      return ea.out && ea.ldo % 8 == 0 && ((uintptr_t)ea.out & 15) == 0;
+    case EPI_RESID_ATTN:
+      return ea.x && ea.x0 && ea.lam && ea.ldr % 8 == 0 &&
+             (((uintptr_t)ea.x | (uintptr_t)ea.x0) & 15) == 0;
+    case EPI_RESID_MLP:
+      return ea.x && ea.lam && ea.ldr % 8 == 0 && ((uintptr_t)ea.x & 15) == 0;
+    case EPI_QKV:
+      return gemm_qkv_fits(M, N, K, ea);
+    case EPI_LOGITS:
+      return !ea.amax && ea.ldz % 8 == 0 && (((uintptr_t)ea.z | (uintptr_t)ea.logits) & 15) == 0;
+    default:
+      return false;
+  }
+}
+
+hipError_t gemm_ring_prepare() {
+  static const bool ok = ring_attrs<EPI_STORE>() && ring_attrs<EPI_RELU2>() &&
+                         ring_attrs<EPI_RESID_ATTN>() && ring_attrs<EPI_RESID_MLP>() &&
+                         ring_attrs<EPI_LOGITS>() && ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
+                         ring_attr<EPI_QKV, 64, 128, 3, 2, 2>() &&
+                         ring_attr<EPI_QKV, 192, 128, 2, 2, 2>();
+  return ok ? hipSuccess : hipErrorInvalidValue;
+}
+
+hipError_t gemm_ring(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                     const EpiArgs& ea, hipStream_t st) {
+  if (!gemm_ring_fits(epi, A, lda, W, M, N, K, ea)) return hipErrorInvalidValue;
+  const hipError_t e = gemm_ring_prepare();
+  if (e != hipSuccess) return e;
+  const int tile = ring_pick(epi, M, N, K);
+#define RING_TILE(E, T, BM, BN, NS, WR, WC) \
+  case T: return launch_ring<E, BM, BN, NS, WR, WC>(A, lda, W, M, N, K, ea, st);
+#define RING(E)                         \
+  switch (tile) {                       \
+    RING_TILE(E, 0, 32, 64, 6, 1, 4)    \
+    RING_TILE(E, 1, 64, 64, 4, 2, 2)    \
+    RING_TILE(E, 2, 128, 64, 3, 2, 2)   \
+    RING_TILE(E, 3, 128, 128, 2, 2, 2)  \
+    RING_TILE(E, 4, 128, 192, 2, 2, 2)  \
+  }                                     \
+  break;
+  switch (epi) {
+    case EPI_STORE: RING(EPI_STORE)
+    case EPI_RELU2: RING(EPI_RELU2)
+    case EPI_RESID_ATTN: RING(EPI_RESID_ATTN)
+    case EPI_RESID_MLP: RING(EPI_RESID_MLP)
+    case EPI_LOGITS: RING(EPI_LOGITS)
+    case EPI_QKV:
+      switch (tile) {
+        RING_TILE(EPI_QKV, 3, 128, 128, 2, 2, 2)
+        RING_TILE(EPI_QKV, 5, 64, 128, 3, 2, 2)
+        RING_TILE(EPI_QKV, 6, 192, 128, 2, 2, 2)
+      }
+  }
+#undef RING
+#undef RING_TILE
+  return hipErrorInvalidValue;
+}
+
+}  // namespace ann

@@ -8,9 +8,10 @@
 //  * k_gemm_sk / k_gemm_sk2: decode projections for 8 < M <= 128 rows on
 //    MFMA, one 16x16 or 32x32 output tile per work-group, K split over the
 //    four waves.
-//  * k_gemm / k_gemm_2w / k_gemm_bat: prefill, wide outputs and batched
-//    products on MFMA (v_mfma_f32_16x16x32_bf16): 64..256 x 128..256 x 64
-//    tiles of four waves, swizzled LDS, register-prefetched K loop.
+//  * k_gemm / k_gemm_2w / k_gemm_bat: the lm_head's loss and top-k forms and
+//    batched products on MFMA (v_mfma_f32_16x16x32_bf16): 64..256 x 64..128 x
+//    64 tiles of four waves, swizzled LDS, register-prefetched K loop.  The
+//    other projections of the prefill are in gemm_ring.hip and gemm_big.hip.
 #include <stdlib.h>
 #include <type_traits>
 #include "common.h"
@@ -527,7 +528,7 @@ __device__ __forceinline__ int gm_lds(int row, int c) {
 
 // Work-group tile BM x BN, four waves of BM/2 x BN/2.  BM = 64 when M <= 64
 // (no padding rows in the MFMAs: the batch-64 lm_head runs 1.4x faster
-// measured), 128 below 512 rows, 256 x 128 / 128 x 256 above (k_gemm_2w).
+// measured), 128 below 512 rows, 256 above (k_gemm_2w).
 // DEPTH: K tiles in flight per thread (a register ring; 1 = the next tile
 // only).  Each K tile of a thread is one memory round trip after the tile
 // before it is stored: with few work-groups and short K loops (decode) a
@@ -541,16 +542,16 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   constexpr int WM = BM / 2, MT = WM / 16;   // rows per wave, 16-row MFMA tiles per wave
   constexpr int WN = BN / 2, NT = WN / 16;   // columns per wave, 16-column tiles per wave
   constexpr int CH = AC > BC ? AC : BC;
-  // the QKV and CE epilogues work on 128-column tiles (whole heads; the
-  // per-tile partial sums of the loss)
-  static_assert((EPI != EPI_QKV && EPI != EPI_CE) || BN == GM_BN, "128-column tiles");
+  // the CE epilogue works on 128-column tiles (the per-tile partial sums of
+  // the loss)
+  static_assert(EPI != EPI_CE || BN == GM_BN, "128-column tiles");
   static_assert(EPI != EPI_TOPK || BN % 128 == 0, "whole 128-column candidate tiles");
-  // staged epilogues (QKV; PE_B / PE_X on full tiles) reuse the LDS for a bf16
+  // staged epilogues (TOPK; PE_B / PE_X on full tiles) reuse the LDS for a bf16
   // BM x BN tile of row pitch BN + 8
   // the batched plain store stages its 128 x 128 tiles for the symmetric form
   constexpr bool STAGE_STORE = EPI == EPI_STORE && BM == GM_BM && BN == GM_BN && DEPTH == 1;
   constexpr bool STAGED =
-      EPI == EPI_QKV || EPI == EPI_PE_B || EPI == EPI_PE_X || EPI == EPI_TOPK || STAGE_STORE;
+      EPI == EPI_PE_B || EPI == EPI_PE_X || EPI == EPI_TOPK || STAGE_STORE;
   constexpr int SMEM = (BM + BN) * GM_BK > (STAGED ? BM * (BN + 8) : 0)
                            ? (BM + BN) * GM_BK
                            : BM * (BN + 8);
@@ -638,9 +639,7 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   // SWAP: acc[j][i] is block (N block j, M block i) of C^T = W A^T, so that a
   // lane holds four consecutive columns n of one row m (8-byte epilogue
   // accesses); otherwise block (M block i, N block j) of C = A W^T, a lane
-  // holding one column of four rows.  Measured: the read-modify-write
-  // epilogues gain from SWAP (prefill o / proj 20 us each), the plain stores
-  // lose (qkv / fc 16 us each).
+  // holding one column of four rows (the plain stores).
   constexpr bool SWAP = EPI != EPI_STORE && EPI != EPI_RELU2;
   floatx4_t acc[NT][MT];
 #pragma unroll
@@ -800,21 +799,6 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
         if (m < M) ea.ce_part[(size_t)tn * ea.ldz + m] = rs[i] + red[wm * WM + i * 16 + r16];
       }
     }
-  } else if constexpr (EPI == EPI_QKV) {
-    QkvRows<BM> pr;
-    qkv_prefetch<BM>(ea, m0, M, tid, pr);
-    __syncthreads();   // every wave is done with the last K tile in LDS
-    constexpr int CP = BN + 8;
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const floatx4_t y = acc[j][i];
-        *(uint2*)(smem + (wm * WM + i * 16 + r16) * CP + wn * WN + j * 16 + (lane >> 4) * 4) =
-            make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
-      }
-    __syncthreads();
-    qkv_tile_epilogue<BM, GM_BN + 8>(ea, smem, m0, n0, M, tid, pr);
   } else if constexpr (EPI == EPI_TOPK) {
     __syncthreads();   // every wave is done with the last K tile in LDS
     constexpr int CP = BN + 8;
@@ -929,11 +913,10 @@ __global__ __launch_bounds__(256) void k_gemm_deep(const bf16_t* __restrict__ A,
   gemm_body<EPI, BM, BN, DEPTH>(A, lda, W, M, N, K, ea);
 }
 
-// The 256 x 128 and 128 x 256 tiles (waves of 128 x 64 / 64 x 128: a quarter
-// less LDS traffic per flop than 64 x 64) held to two waves per SIMD, so two
-// work-groups share a CU.  Measured 10-15% faster than 128 x 128 on the
-// prefill shapes; without the register cap the compiler takes one wave per
-// SIMD and they are slower.
+// The 256 x 128 tile (waves of 128 x 64: a quarter less LDS traffic per flop
+// than 64 x 64) held to two waves per SIMD, so two work-groups share a CU.
+// Measured 10-15% faster than 128 x 128; without the register cap the
+// compiler takes one wave per SIMD and it is slower.
 template <int EPI, int BM, int BN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_2w(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int M, int N, int K,
@@ -1359,48 +1342,36 @@ hipError_t gemm_decode64(int epi, const bf16_t* A, int lda, const bf16_t* W, int
 hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                 const EpiArgs& ea, hipStream_t st) {
   if (K % GM_BK != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  // large shapes of the epilogues where it measured faster: the 256 x 256
-  // one-work-group-per-CU kernel (gemm_big.hip).  ANN_GEMM_BIG=0 keeps every
-  // shape on the tiles below, ANN_GEMM_BIG=2 sends every epilogue it takes
-  // there (read at every call)
-  const char* big_env = getenv("ANN_GEMM_BIG");
-  const int big_mode = big_env ? atoi(big_env) : 1;
-  if (big_mode != 0 && (big_mode == 2 || gemm_big_routes(epi, M, N)) &&
-      gemm_big_fits(epi, A, lda, M, N, K, ea)) {
-    if (epi == EPI_QKV && !gemm_qkv_fits(M, N, K, ea)) return hipErrorInvalidValue;
-    return gemm_big(epi, A, lda, W, M, N, K, ea, st);
+  // the MLP's output projection of a large input: the 256 x 256 one-work-
+  // group-per-CU kernel (gemm_big.hip).  ANN_GEMM_BIG=0 keeps it on the ring
+  // kernel, ANN_GEMM_BIG=2 sends every shape it takes there (read at every
+  // call)
+  if (epi == EPI_RESID_MLP) {
+    const char* big_env = getenv("ANN_GEMM_BIG");
+    const int big_mode = big_env ? atoi(big_env) : 1;
+    if (big_mode != 0 && (big_mode == 2 || gemm_big_routes(M, K)) &&
+        gemm_big_fits(A, lda, M, N, K, ea))
+      return gemm_big(A, lda, W, M, N, K, ea, st);
   }
-  // tile: 64 x 128 for at most 64 rows; 128 x 128 below 512 rows; then
-  // 256 x 128 (wide outputs, and the 128-column QKV / CE epilogues) or
-  // 128 x 256 (outputs of at most 1024 columns: the o / proj projections)
-  const int shape = M <= 64 ? 0 : M < 512 ? 1
-                  : (epi == EPI_QKV || epi == EPI_CE || N > 1024) ? 2 : 3;
+  if (gemm_ring_fits(epi, A, lda, W, M, N, K, ea)) return gemm_ring(epi, A, lda, W, M, N, K, ea, st);
+  // what the ring kernel does not take (the CE and top-k epilogues, a
+  // vocabulary that is no multiple of 64): 64 x 128 tiles for at most 64 rows,
+  // 128 x 128 below 512 rows, then 256 x 128
+  const int shape = M <= 64 ? 0 : M < 512 ? 1 : 2;
   const int bm = shape == 0 ? 64 : shape == 2 ? 256 : 128;
-  const int bn = shape == 3 ? 256 : GM_BN;
-  dim3 grid((N + bn - 1) / bn, (M + bm - 1) / bm);
+  dim3 grid((N + GM_BN - 1) / GM_BN, (M + bm - 1) / bm);
 #define ANN_GM_ONE(E, S)                                                                       \
   if (S == 0)                                                                                  \
     hipLaunchKernelGGL((k_gemm<E, 64, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K, ea); \
   else if (S == 1)                                                                             \
     hipLaunchKernelGGL((k_gemm<E, 128, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K,    \
                        ea);                                                                    \
-  else if (S == 2)                                                                             \
+  else                                                                                         \
     hipLaunchKernelGGL((k_gemm_2w<E, 256, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K, \
                        ea);
-#define ANN_GM(E)                                                                              \
-  ANN_GM_ONE(E, shape)                                                                         \
-  else hipLaunchKernelGGL((k_gemm_2w<E, 128, 256>), grid, dim3(256), 0, st, A, lda, W, M, N,   \
-                          K, ea);                                                              \
-  break;
   switch (epi) {
-    case EPI_STORE: ANN_GM(EPI_STORE)
-    case EPI_RELU2: ANN_GM(EPI_RELU2)
-    case EPI_RESID_ATTN: ANN_GM(EPI_RESID_ATTN)
-    case EPI_RESID_MLP: ANN_GM(EPI_RESID_MLP)
-    case EPI_LOGITS: ANN_GM(EPI_LOGITS)
-    case EPI_QKV:
-      if (!gemm_qkv_fits(M, N, K, ea)) return hipErrorInvalidValue;
-      ANN_GM_ONE(EPI_QKV, shape)
+    case EPI_LOGITS:
+      ANN_GM_ONE(EPI_LOGITS, shape)
       break;
     case EPI_CE:
       if (!ea.ce_part || !ea.ce_tz || !ea.tgt || ea.ldz < M) return hipErrorInvalidValue;
@@ -1411,13 +1382,17 @@ hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N
       if (shape > 1 || !ea.cand || !ea.cand_r || ea.nt != (N + 127) / 128 || ea.Vs < 1 ||
           ea.Vs > N || N > 65536 || (ea.logits && ea.ldz < N))
         return hipErrorInvalidValue;
-      ANN_GM_ONE(EPI_TOPK, shape)
+      if (shape == 0)
+        hipLaunchKernelGGL((k_gemm<EPI_TOPK, 64, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N,
+                           K, ea);
+      else
+        hipLaunchKernelGGL((k_gemm<EPI_TOPK, 128, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N,
+                           K, ea);
       break;
     }
     default:
       return hipErrorInvalidValue;
   }
-#undef ANN_GM
 #undef ANN_GM_ONE
   return hipGetLastError();
 }
