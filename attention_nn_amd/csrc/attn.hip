@@ -15,10 +15,13 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 // ---- prefill: MFMA flash attention ------------------------------------------
 //
-// Grid (ceil(T/128), H, B), 512 threads: 8 waves x 16 queries.  K and V tiles
-// of BK keys stream through a ring of NS LDS stages: each tile is loaded
-// straight into LDS (global_load_lds_dwordx4, 1 KB per wave instruction, no
-// register staging) NS - 1 tiles ahead of its use; one barrier per tile.  LDS
+// Grid (ceil(T/BQ), H, B), 512 threads: 8 waves in KP key parts of 8 / KP waves
+// x 16 queries (BQ = 128 / KP).  A ring stage holds KP tiles of BK keys, one
+// for each part; with KP > 1 the parts' sums are added through LDS at the end
+// (the fixed softmax shift leaves nothing to rescale).  K and V tiles stream
+// through a ring of NS LDS stages: each tile is loaded straight into LDS
+// (global_load_lds_dwordx4, 1 KB per wave instruction, no register staging)
+// NS - 1 stages ahead of its use; one barrier per stage.  LDS
 // rows are the unpadded DH-element rows of the cache with 16-byte chunk c of
 // row r stored at chunk c ^ swz(r), conflict-free on the 64 banks for both
 // fragment reads below.  Each wave computes S^T = K Q^T with
@@ -88,22 +91,30 @@ __device__ __forceinline__ void ap_static_for(F&& f) {
   }
 }
 
-template <int DH, int BK, int NS>
-constexpr size_t ap_lds_bytes() { return (size_t)NS * 2 * BK * DH * 2; }
+// the ring, or the partial sums of KP - 1 key parts (fp32, their row pitch
+// DH + 4 words)
+template <int DH, int BK, int NS, int KP>
+constexpr size_t ap_lds_bytes() {
+  const size_t ring = (size_t)NS * KP * 2 * BK * DH * 2;
+  const size_t sums = (size_t)(KP - 1) * (128 / KP) * (DH + 4) * 4;
+  return ring > sums ? ring : sums;
+}
 
 // two work-groups per CU (four waves per SIMD, 128 VGPRs) where their rings
 // fit the 160 KB of LDS together, else one (256 VGPRs)
-template <int DH, int BK, int NS>
-constexpr int ap_waves_per_eu() { return ap_lds_bytes<DH, BK, NS>() <= 80 * 1024 ? 4 : 2; }
+template <int DH, int BK, int NS, int KP>
+constexpr int ap_waves_per_eu() { return ap_lds_bytes<DH, BK, NS, KP>() <= 80 * 1024 ? 4 : 2; }
 
-template <int DH, int BK, int NS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_per_eu<DH, BK, NS>()))) void k_attn_prefill(
+template <int DH, int BK, int NS, int KP>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_per_eu<DH, BK, NS, KP>()))) void k_attn_prefill(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int32_t* __restrict__ pos, bf16_t* __restrict__ out, int T, int H, int max_ctx,
     int window, int is_long, float scale, float shift, int lpt) {
-  constexpr int BQ = 128;
+  constexpr int QW = 8 / KP;          // waves across the queries
+  constexpr int BQ = 16 * QW;
+  constexpr int SK = BK * KP;         // keys of a ring stage: one tile per key part
   constexpr int RB = DH * 2;          // LDS row bytes
-  constexpr int TB = BK * RB;         // bytes of one K (or V) tile
+  constexpr int TB = SK * RB;         // bytes of a stage's K (or V) rows
   constexpr int LPW = TB / 1024 / 8;  // 1 KB load instructions per wave per K (or V) tile
   static_assert(LPW >= 1 && LPW * 8 * 1024 == TB, "tile split over the waves");
   static_assert(NS >= 2 && NS <= 6, "ring depth");
@@ -141,18 +152,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
       b = w / (nx * ny);
     }
   }
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qw = wv % QW, kp = wv / QW;   // this wave's queries and key part
   const int r16 = lane & 15, g4 = lane >> 4;
   const int d = H * DH;
   const int p0 = pos[b];
   const int qs = qb * BQ;
-  const int tq = qs + wv * 16 + r16;   // this lane's query (B-operand column)
+  const int tq = qs + qw * 16 + r16;   // this lane's query (B-operand column)
   const bool qok = tq < T;
   const int qp = p0 + tq;              // its position
   // this wave's 16 queries: positions wq0 .. wq0 + 15 (all valid iff wall)
-  const int wq0 = p0 + qs + wv * 16;
-  const bool wall = qs + wv * 16 + 15 < T;
-  const int wqn = min(T - (qs + wv * 16), 16);   // valid queries of the wave (may be <= 0)
+  const int wq0 = p0 + qs + qw * 16;
+  const bool wall = qs + qw * 16 + 15 < T;
+  const int wqn = min(T - (qs + qw * 16), 16);   // valid queries of the wave (may be <= 0)
 
   // q fragments: unconditional loads issued ahead of the ring's (a query past
   // T reads row T - 1: its scores are always masked and its output not stored)
@@ -166,7 +179,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
   const int klo = is_long ? 0 : max(0, qpos_lo - window + 1);
   const int kbeg = klo & ~(BK - 1);
   const int kend = qpos_hi + 1;
-  const int ntile = (kend - kbeg + BK - 1) / BK;
+  const int ntile = (kend - kbeg + SK - 1) / SK;   // ring stages
   const size_t head = ((size_t)b * H + h) * max_ctx;
   const bf16_t* kh = kc + head * DH;
   const bf16_t* vh = vc + head * DH;
@@ -182,7 +195,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
     lcol[u] = (((o % RB) >> 4) ^ ap_swz<DH>(o / RB)) * 8;
   }
   auto issue = [&](int t) {
-    const int kb = kbeg + t * BK;
+    const int kb = kbeg + t * SK;
     unsigned char* st = ap_smem + (size_t)(t % NS) * 2 * TB;
 #pragma unroll
     for (int u = 0; u < LPW; ++u) {
@@ -216,7 +229,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t) issue(t);
   for (int t = 0; t < ntile; ++t) {
-    const int kb = kbeg + t * BK;
+    const int kb = kbeg + t * SK + kp * BK;   // this wave's tile of the stage
     wait_tiles(min(NS - 2, ntile - 1 - t));   // this wave's part of tile t is in LDS
     __syncthreads();                            // every wave's; stage (t - 1) % NS is free
     if (t + NS - 1 < ntile) issue(t + NS - 1);
@@ -225,7 +238,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
     const bool live = wqn > 0 && kb <= wq0 + wqn - 1 && (is_long || wq0 - (kb + BK - 1) < window);
     if (!live) continue;
     const bool full = wall && kb + BK - 1 <= wq0 && (is_long || wq0 + 15 - kb < window);
-    const unsigned char* ks_ = ap_smem + (size_t)(t % NS) * 2 * TB;
+    const unsigned char* ks_ = ap_smem + (size_t)(t % NS) * 2 * TB + kp * BK * RB;
     const unsigned char* vs_ = ks_ + TB;
 
     ap_lds_cchar* kst = (ap_lds_cchar*)ks_ + r16 * RB;
@@ -308,6 +321,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
   ap_wait_vm<0>();   // no load into LDS outlives the work-group
   lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
+  if constexpr (KP > 1) {
+    // the key parts' sums, added in part order (one fixed softmax shift, so
+    // nothing is rescaled): parts 1 .. KP - 1 leave theirs in LDS
+    constexpr int PW = DH + 4;
+    float* sums = (float*)ap_smem;
+    __syncthreads();   // every wave is done with the ring
+    if (kp > 0) {
+      float* row = sums + ((kp - 1) * BQ + qw * 16 + r16) * PW;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) *(floatx4_t*)(row + db * 16 + g4 * 4) = o[db];
+      if (g4 == 0) row[DH] = lsum;
+    }
+    __syncthreads();
+    if (kp > 0) return;
+#pragma unroll
+    for (int part = 1; part < KP; ++part) {
+      const float* row = sums + ((part - 1) * BQ + qw * 16 + r16) * PW;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) o[db] += *(const floatx4_t*)(row + db * 16 + g4 * 4);
+      lsum += row[DH];
+    }
+  }
   if (qok) {
     const float inv = 1.f / lsum;
     bf16_t* orow = out + (size_t)(b * T + tq) * d + h * DH;
@@ -321,30 +356,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(ap_waves_pe
   }
 }
 
-template <int DH, int BK, int NS>
-static hipError_t attn_prefill_launch(dim3 grid, hipStream_t st, const bf16_t* q, const bf16_t* kc,
-                                      const bf16_t* vc, const int32_t* pos, bf16_t* out, int T,
-                                      int H, int max_ctx, int window, bool long_layer, float scale,
-                                      float shift) {
-  constexpr size_t lds = ap_lds_bytes<DH, BK, NS>();
-  static hipError_t attr = hipFuncSetAttribute((const void*)k_attn_prefill<DH, BK, NS>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+template <int DH, int BK, int NS, int KP>
+static hipError_t attn_prefill_launch(hipStream_t st, const bf16_t* q, const bf16_t* kc,
+                                      const bf16_t* vc, const int32_t* pos, bf16_t* out, int B,
+                                      int T, int H, int max_ctx, int window, bool long_layer,
+                                      float scale, float shift, int cus) {
+  constexpr size_t lds = ap_lds_bytes<DH, BK, NS, KP>();
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)k_attn_prefill<DH, BK, NS, KP>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
+  constexpr int BQ = 128 / KP;
+  const dim3 grid((T + BQ - 1) / BQ, H, B);
   // longest query blocks first when one block's (row, head) pairs fit the
   // resident work-groups (ap_waves_per_eu: 4 waves per SIMD = two 8-wave
   // work-groups per CU, else one)
-  static int cus = 0;
-  if (!cus) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-  }
-  const long long resident = (long long)cus * (ap_waves_per_eu<DH, BK, NS>() / 2);
+  const long long resident = (long long)cus * (ap_waves_per_eu<DH, BK, NS, KP>() / 2);
   const int lpt = (long long)grid.y * grid.z <= resident ? 1 : 0;
-  hipLaunchKernelGGL((k_attn_prefill<DH, BK, NS>), grid, dim3(512), lds, st, q, kc, vc, pos, out, T,
-                     H, max_ctx, window, (int)long_layer, scale, shift, lpt);
+  hipLaunchKernelGGL((k_attn_prefill<DH, BK, NS, KP>), grid, dim3(512), lds, st, q, kc, vc, pos,
+                     out, T, H, max_ctx, window, (int)long_layer, scale, shift, lpt);
   return hipGetLastError();
 }
 
@@ -352,20 +382,32 @@ hipError_t attn_prefill(const bf16_t* q, const bf16_t* kc, const bf16_t* vc, con
                         bf16_t* out, int B, int T, int H, int Dh, int max_ctx, int window,
                         bool long_layer, float scale, hipStream_t st) {
   if (B <= 0 || T <= 0) return hipErrorInvalidValue;
+  static const int cus = device_cus();
   const float shift = scale * (float)Dh * 1.02f;
-  dim3 grid((T + 127) / 128, H, B);
-  // ring of two 32-key stages: deeper rings (3 to 5 stages, or 64-key tiles
-  // with one work-group per CU) measured equal or slower
-#define AP_ARGS grid, st, q, kc, vc, pos, out, T, H, max_ctx, window, long_layer, scale, shift
-  switch (Dh) {
-    case 64:
-      return attn_prefill_launch<64, 64, 2>(AP_ARGS);
-    case 128:
-      return attn_prefill_launch<128, 32, 2>(AP_ARGS);
-    default:
-      return hipErrorInvalidValue;
+  // Key parts: a work-group of 128 queries walks its keys in tiles of 32, about
+  // 1 us each, so where those work-groups leave CUs idle a work-group takes 128
+  // / kp queries and kp tiles at a time.  155M prefill, us for the whole call
+  // with kp 1 / 2 / 4: 777 tokens (42 work-groups of 128 queries) 735 / 660 /
+  // 636, 2 x 777 (84) 983 / 914 / 917, 4 x 777 (168) 1262 / 1202 / 1267, 8 x 777
+  // (336) 2021 / 2018 / 2180, 16 x 777 3183 / 3208 / 3605; head dim 64, 777
+  // tokens (56) 371 / 347 / 328, 4 x 777 (224) 580 / 562 / 630.
+  const long long wgs = (long long)((T + 127) / 128) * H * B;
+  const int kp = 4 * wgs <= cus ? 4 : wgs <= cus ? 2 : 1;
+  // ring of two stages: deeper ones (three or four, or 64-key tiles with one
+  // work-group per CU) measured equal or slower, at small grids too
+#define AP_ARGS st, q, kc, vc, pos, out, B, T, H, max_ctx, window, long_layer, scale, shift, cus
+  if (Dh == 64) {
+    if (kp == 4) return attn_prefill_launch<64, 64, 2, 4>(AP_ARGS);
+    if (kp == 2) return attn_prefill_launch<64, 64, 2, 2>(AP_ARGS);
+    return attn_prefill_launch<64, 64, 2, 1>(AP_ARGS);
+  }
+  if (Dh == 128) {
+    if (kp == 4) return attn_prefill_launch<128, 32, 2, 4>(AP_ARGS);
+    if (kp == 2) return attn_prefill_launch<128, 32, 2, 2>(AP_ARGS);
+    return attn_prefill_launch<128, 32, 2, 1>(AP_ARGS);
   }
 #undef AP_ARGS
+  return hipErrorInvalidValue;
 }
 
 }  // namespace ann
