@@ -84,7 +84,8 @@ size_t pd_layout(const ann_config& c, int which) {
   return ann::pd_layout((size_t)c.d, (size_t)c.H, which);
 }
 
-// 128-column tiles of the lm_head GEMM (its work-group tile width).
+// 128-column tiles of the lm_head (the top-k records; at most that many
+// partial sums per row of the loss).
 int ce_tiles(const ann_config& c) { return (c.V + 127) / 128; }
 
 SLayout ws_layout(const ann_config& c) {
@@ -273,6 +274,14 @@ int proj(ann_ctx* c, int kind, int epi, int pre, const bf16_t* W, const bf16_t* 
   const bool use_gemv = !gemm_only && gemv_routes(M, K);
   const bool use_sk = !gemm_only && !use_gemv && !proj_is_gemm(M, N, K, pre);
   if (epi == EPI_QKV && (use_gemv || use_sk)) return fail(ANN_E_ARG, "fused QKV needs the MFMA GEMM");
+  ea.eps = c->c.rms_eps;
+  // a small tile of the ring GEMM forms rms(X) @ W^T from X itself
+  if (pre == PRE_RMS && !use_gemv && !use_sk && gemm_ring_fits(epi, X, ldx, W, M, N, K, ea) &&
+      gemm_ring_rms(epi, M, N, K)) {
+    ProfScope ps(c, kind, st);
+    HIPCHK(gemm_ring(epi, X, ldx, W, M, N, K, ea, st));
+    return ANN_OK;
+  }
   // 65-128 rows with an RMS prologue and a plain-store epilogue (qkv, fc):
   // rms_apply + 64 x 64 MFMA tiles beat the skinny kernel's in-kernel RMS
   // (cfg5 decode 3.99 -> 3.88 ms per step, measured); up to 64 rows the
@@ -1004,7 +1013,9 @@ int ann_forward_loss(ann_ctx* c, const int32_t* tokens, const int32_t* targets, 
             c->c.d, M, c->c.V, c->c.d, ec, st);
   if (rc) return rc;
   float* rows = row_loss ? row_loss : c->sp<float>(c->sl.ce_rows);
-  HIPCHK(ce_finalize(ec.ce_part, M, ce_tiles(c->c), ec.ce_tz, M, rows, loss, st));
+  const int cols = gemm_ce_cols(c->sp<bf16_t>(c->sl.hn), c->c.d, c->wptr(c->wl.head), M, c->c.V,
+                                c->c.d, ec);
+  HIPCHK(ce_finalize(ec.ce_part, M, (c->c.V + cols - 1) / cols, ec.ce_tz, M, rows, loss, st));
   HIPCHK(advance_pos(pos, B, T, st));
   c->len = T;
   return ANN_OK;

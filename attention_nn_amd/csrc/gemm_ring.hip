@@ -32,7 +32,18 @@ constexpr int RG_RB = RG_BK * 2;   // bytes of an LDS row
 typedef __bf16 rg_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float rg_floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t rg_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 rg_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void rg_lds_void;
+
+// c + the sum of squares of a fragment's eight values (v_dot2_f32_bf16)
+__device__ __forceinline__ float rg_sumsq(const rg_bf16x8& a, float c) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const rg_bf16x2 v = {a[e], a[e + 1]};
+    c = __builtin_amdgcn_fdot2_f32_bf16(v, v, c, false);
+  }
+  return c;
+}
 
 template <int I, int N, typename F>
 __device__ __forceinline__ void rg_static_for(F&& f) {
@@ -47,6 +58,11 @@ __device__ __forceinline__ void rg_static_for(F&& f) {
 template <int N>
 __device__ __forceinline__ void rg_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+}
+
+// Whether a tile forms rms(A) @ W^T from A itself.
+constexpr bool ring_takes_rms(int epi, int bm, int bn) {
+  return (epi == EPI_STORE || epi == EPI_RELU2 || epi == EPI_QKV) && bm * bn <= 128 * 64;
 }
 
 template <int BM, int BN, int NS>
@@ -72,6 +88,15 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
   // the residual operands: loaded first where the tile is small (a few
   // registers, and nothing else hides the latency), after the main loop else
   constexpr bool EARLY = RES && BM * BN <= 128 * 64;
+  // the qkv and fc projections are of rms(x).  The small tiles take x itself
+  // as A and scale y by the row's rsqrt(mean(x^2) + eps) after the product; the
+  // sums of squares come from the A fragments on their way to the MFMAs (four
+  // dot instructions each), so that no launch normalises a copy first: 155M
+  // prompts of 777 / 300 tokens 690 -> 647 and 594 -> 547 us.  The large tiles
+  // have no issue slots for that (d 1536, 128 x 1024 tokens and 24 steps: 36.55
+  // ms with it, 35.80 without).  The lm_head always takes the
+  // rounded rms(x), so that z is the same bits on every route to it.
+  constexpr bool RMS = ring_takes_rms(EPI, BM, BN);
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && BM * CPR % TH == 0, "whole loads");
   static_assert(EPI != EPI_QKV || (BN == 128 && TH == 256), "whole heads per tile");
   extern __shared__ __attribute__((aligned(16))) unsigned char rg_smem[];
@@ -144,6 +169,9 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     }
   };
 
+  float ss[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) ss[i] = 0.f;
   rg_floatx4 acc[NT][MT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -172,10 +200,12 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
+      for (int i = 0; i < MT; ++i) {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
           acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h][j], a[h][i], acc[j][i], 0, 0, 0);
+        if constexpr (RMS) ss[i] = rg_sumsq(a[h][i], ss[i]);
+      }
   };
 
   // ring: K tile t in stage t % NS, loaded NS - 1 tiles ahead.  The barrier
@@ -197,6 +227,63 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     s = s + 1 == NS ? 0 : s + 1;
   });
 
+  if constexpr (RMS) {
+    // a lane's column of C^T is row r16 of its M blocks, whose squares the four
+    // lanes of that r16 have summed
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      float t = ss[i];
+      t += __shfl_xor(t, 16, 64);
+      t += __shfl_xor(t, 32, 64);
+      const float f = rsqrtf(t / (float)K + ea.eps);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j][i] *= f;
+    }
+  }
+  if constexpr (EPI == EPI_CE) {
+    // softcap(bf16(z)) in (0, 23): sum exp(zc) needs no max pass.  Row sums:
+    // in-lane over the wave's N blocks, then over the four lane groups, then
+    // the column parts through LDS, always in the same order.  Hardware exp2
+    // and reciprocal: the IEEE expf and division cost ~35 VALU instructions
+    // per logit.
+    float* red = (float*)rg_smem;
+    float rs[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wm * WM + i * 16 + r16;
+      const int tg = m < M ? ea.tgt[m] : -1;
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int n = n0 + wn * WN + j * 16 + kg * 4 + r;
+          const float zc = softcap_fast(rbf(acc[j][i][r]));
+          sum += __builtin_amdgcn_exp2f(zc * 1.4426950408889634f);
+          if (n == tg) ea.ce_tz[m] = zc;
+        }
+      sum += __shfl_xor(sum, 16, 64);
+      sum += __shfl_xor(sum, 32, 64);
+      rs[i] = sum;
+    }
+    __syncthreads();   // every wave is done with the last K tile
+    if (wn > 0 && kg == 0) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) red[(wn - 1) * BM + wm * WM + i * 16 + r16] = rs[i];
+    }
+    __syncthreads();
+    if (wn == 0 && kg == 0) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const int ml = wm * WM + i * 16 + r16;
+        float t = rs[i];
+#pragma unroll
+        for (int p = 0; p < WC - 1; ++p) t += red[p * BM + ml];
+        if (m0 + ml < M) ea.ce_part[(size_t)tn * ea.ldz + m0 + ml] = t;
+      }
+    }
+    return;
+  }
   // epilogue: bf16(y) staged in LDS, then 16-byte row chunks
   if constexpr (RES && !EARLY) res_load();
   QkvRows<BM> pr;
@@ -316,6 +403,7 @@ static int ring_pick(int epi, int M, int N, int K) {
   for (int i = 0; i < RING_QKV_N; ++i) {
     const RingTile& t = RING_TILES[i];
     if (epi == EPI_QKV ? t.bn != 128 : i >= RING_N) continue;
+    if (epi == EPI_CE && t.bn < 128) continue;   // partial sums of at most V / 128 tiles
     if (N % t.bn) continue;
     const long long wgs = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn);
     const long long n = (wgs + cus - 1) / cus;
@@ -346,6 +434,8 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
       return ea.x && ea.lam && ea.ldr % 8 == 0 && ((uintptr_t)ea.x & 15) == 0;
     case EPI_QKV:
       return gemm_qkv_fits(M, N, K, ea);
+    case EPI_CE:
+      return (N % 128 == 0 || N % 192 == 0) && ea.ce_part && ea.ce_tz && ea.tgt && ea.ldz >= M;
     case EPI_LOGITS:
       return !ea.amax && ea.ldz % 8 == 0 && (((uintptr_t)ea.z | (uintptr_t)ea.logits) & 15) == 0;
     default:
@@ -353,10 +443,22 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
   }
 }
 
+int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                 const EpiArgs& ea) {
+  return gemm_ring_fits(EPI_CE, A, lda, W, M, N, K, ea) ? RING_TILES[ring_pick(EPI_CE, M, N, K)].bn
+                                                        : 128;
+}
+
+bool gemm_ring_rms(int epi, int M, int N, int K) {
+  const RingTile& t = RING_TILES[ring_pick(epi, M, N, K)];
+  return ring_takes_rms(epi, t.bm, t.bn);
+}
+
 hipError_t gemm_ring_prepare() {
   static const bool ok = ring_attrs<EPI_STORE>() && ring_attrs<EPI_RELU2>() &&
                          ring_attrs<EPI_RESID_ATTN>() && ring_attrs<EPI_RESID_MLP>() &&
-                         ring_attrs<EPI_LOGITS>() && ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
+                         ring_attrs<EPI_LOGITS>() && ring_attr<EPI_CE, 128, 128, 2, 2, 2>() &&
+                         ring_attr<EPI_CE, 128, 192, 2, 2, 2>() && ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
                          ring_attr<EPI_QKV, 64, 128, 3, 2, 2>() &&
                          ring_attr<EPI_QKV, 192, 128, 2, 2, 2>();
   return ok ? hipSuccess : hipErrorInvalidValue;
@@ -385,6 +487,12 @@ hipError_t gemm_ring(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, 
     case EPI_RESID_ATTN: RING(EPI_RESID_ATTN)
     case EPI_RESID_MLP: RING(EPI_RESID_MLP)
     case EPI_LOGITS: RING(EPI_LOGITS)
+    case EPI_CE:
+      switch (tile) {
+        RING_TILE(EPI_CE, 3, 128, 128, 2, 2, 2)
+        RING_TILE(EPI_CE, 4, 128, 192, 2, 2, 2)
+      }
+      break;
     case EPI_QKV:
       switch (tile) {
         RING_TILE(EPI_QKV, 3, 128, 128, 2, 2, 2)

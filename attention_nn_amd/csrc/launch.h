@@ -18,7 +18,7 @@ namespace ann {
 //                   and v = bf16(y_v) -> the KV cache at [b][h][pos[b] + t]
 //                   (model.py:244-247, 252)
 //   EPI_CE          (MFMA GEMM only, lm_head of the training forward) per row m and
-//                   128-column tile t: ce_part[t * ldz + m] = sum of exp(softcap(bf16(y)))
+//                   column tile t (gemm_ce_cols): ce_part[t * ldz + m] = sum of exp(softcap(bf16(y)))
 //                   over the tile's columns; ce_tz[m] = softcap(bf16(y[tgt[m]])) from
 //                   the tile holding the target (metal_kernels.py:153-193)
 //   EPI_TOPK        (MFMA GEMM only, decode lm_head of 3..511 rows) per row m and
@@ -122,11 +122,18 @@ bool gemm_qkv_fits(int M, int N, int K, const EpiArgs& ea);
 // PE_B, PE_X; sOut / sX are the batch strides of ea.out / ea.x.
 // Projections of the prefill, the training forward and whole-context logits:
 // 32 x 64 .. 128 x 192 tiles by shape, K tiles streamed into an LDS ring
-// (gemm_ring.hip).  EPI_STORE, EPI_RELU2, EPI_RESID_*, EPI_QKV, EPI_LOGITS.
+// (gemm_ring.hip).  y = a @ W^T; where gemm_ring_rms says so (EPI_STORE,
+// EPI_RELU2 and EPI_QKV on the small tiles) y = rms(a) @ W^T over rows of K
+// values (ea.eps).
 bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                     const EpiArgs& ea);
+bool gemm_ring_rms(int epi, int M, int N, int K);
 hipError_t gemm_ring(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                      const EpiArgs& ea, hipStream_t st);
+// Columns of gemm_ring's EPI_CE tiles (of gemm()'s, 128, where the ring does
+// not fit): ceil(N / columns) partial sums per row.
+int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                 const EpiArgs& ea);
 // One-time set-up (dynamic LDS limits), called by the entry points before
 // anything they may capture into a graph.
 hipError_t gemm_ring_prepare();
@@ -170,7 +177,8 @@ hipError_t gemm_skinny(int epi, bool rms, const bf16_t* A, int lda, const bf16_t
                        int K, float eps, const EpiArgs& ea, hipStream_t st);
 hipError_t gemm_decode64(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                          const EpiArgs& ea, hipStream_t st);
-// MFMA GEMM (prefill): y = A @ W^T with A (M, lda) bf16.
+// MFMA GEMM: y = A @ W^T with A (M, lda) bf16 (as gemm_ring where that takes
+// the shape).
 hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                 const EpiArgs& ea, hipStream_t st);
 // h = bf16(rms(x)) for M rows of length d (row strides ldx / ldh).

@@ -1354,8 +1354,8 @@ hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N
       return gemm_big(A, lda, W, M, N, K, ea, st);
   }
   if (gemm_ring_fits(epi, A, lda, W, M, N, K, ea)) return gemm_ring(epi, A, lda, W, M, N, K, ea, st);
-  // what the ring kernel does not take (the CE and top-k epilogues, a
-  // vocabulary that is no multiple of 64): 64 x 128 tiles for at most 64 rows,
+  // what the ring kernel does not take (the top-k epilogue, a vocabulary that
+  // is no multiple of 64): 64 x 128 tiles for at most 64 rows,
   // 128 x 128 below 512 rows, then 256 x 128
   const int shape = M <= 64 ? 0 : M < 512 ? 1 : 2;
   const int bm = shape == 0 ? 64 : shape == 2 ? 256 : 128;
