@@ -73,6 +73,113 @@ constexpr size_t rg_lds_bytes() {
 
 }  // namespace
 
+// acc = the (m0, n0) tile of C^T = W A^T: block (N block j, M block i), so that a
+// lane holds four consecutive columns of one row; ss (SQ): this lane's part of
+// the sums of squares of the A rows (row r16 of M block i, summed over the
+// four lanes of that r16).  W is (N, K).  LDS from rg_smem's start; a barrier
+// has to follow before it is written again.
+template <int BM, int BN, int NS, int WR, int WC, bool SQ>
+__device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf16_t* W, int M,
+                                             int N, int K, int m0, int n0, int wv, int lane,
+                                             rg_floatx4 (&acc)[BN / WC / 16][BM / WR / 16],
+                                             float (&ss)[BM / WR / 16]) {
+  constexpr int NW = WR * WC;
+  constexpr int WM = BM / WR, MT = WM / 16;
+  constexpr int WN = BN / WC, NT = WN / 16;
+  constexpr int LA = BM / 8 / NW, LW = BN / 8 / NW;   // 1 KB loads per wave per K tile
+  constexpr int SB = (BM + BN) * RG_RB;               // bytes of a stage
+  extern __shared__ __attribute__((aligned(16))) unsigned char rg_smem[];
+  // load u of this wave fills rows 8 (NW u + wv) .. + 7 of the operand's tile
+  // in LDS: lane l row l >> 3, slot l & 7, which holds logical 16-byte chunk
+  // (l & 7) ^ ((row >> 1) & 7) -- conflict-free for the 16-row fragment reads.
+  // Rows past M / N repeat the last one (they feed outputs never stored).
+  const bf16_t* pa[LA];
+  const bf16_t* pw[LW];
+  const int KT = K / RG_BK;
+#pragma unroll
+  for (int u = 0; u < LA; ++u) {
+    const int r = 8 * (NW * u + wv) + (lane >> 3);
+    pa[u] = A + (size_t)min(m0 + r, M - 1) * lda + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+  }
+#pragma unroll
+  for (int u = 0; u < LW; ++u) {
+    const int r = 8 * (NW * u + wv) + (lane >> 3);
+    pw[u] = W + (size_t)min(n0 + r, N - 1) * K + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+  }
+  // (the builtin's operands have plain types: clang's host pass drops a kernel
+  // in which a type-dependent call of its 16-byte form is instantiated)
+  auto issue = [&](int kt, int s) {
+    unsigned char* st = rg_smem + s * SB;
+#pragma unroll
+    for (int u = 0; u < LA; ++u) {
+      const bf16_t* src = pa[u] + kt * RG_BK;
+      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
+    }
+    st += BM * RG_RB;
+#pragma unroll
+    for (int u = 0; u < LW; ++u) {
+      const bf16_t* src = pw[u] + kt * RG_BK;
+      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
+    }
+  };
+
+#pragma unroll
+  for (int i = 0; i < MT; ++i) ss[i] = 0.f;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[j][i] = (rg_floatx4){0.f, 0.f, 0.f, 0.f};
+
+  // the k steps of 32 run in order, as in every GEMM here: the same bits
+  // whatever the tile
+  const int r16 = lane & 15, kg = lane >> 4, sw = (r16 >> 1) & 7;
+  const int wm = wv / WC, wn = wv % WC;
+  const int oa = (wm * WM + r16) * RG_RB, ow = BM * RG_RB + (wn * WN + r16) * RG_RB;
+  const int c0 = (kg ^ sw) << 4, c1 = ((4 + kg) ^ sw) << 4;
+  auto compute = [&](int s) {
+    const unsigned char* st = rg_smem + s * SB;
+    rg_bf16x8 a[2][MT], w[2][NT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        w[h][j] = *(const rg_bf16x8*)(st + ow + j * 16 * RG_RB + (h ? c1 : c0));
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        a[h][i] = *(const rg_bf16x8*)(st + oa + i * 16 * RG_RB + (h ? c1 : c0));
+    }
+    __builtin_amdgcn_sched_barrier(0);   // all reads in flight, then the MFMAs
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h][j], a[h][i], acc[j][i], 0, 0, 0);
+        if constexpr (SQ) ss[i] = rg_sumsq(a[h][i], ss[i]);
+      }
+  };
+
+  // ring: K tile t in stage t % NS, loaded NS - 1 tiles ahead.  The barrier
+  // that follows the wait for tile t also says that every wave is done with
+  // the stage of tile t - 1, which tile t + NS - 1 then overwrites.  (With
+  // fewer K tiles than that the last one is loaded again, and not used.)
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t) issue(min(t, KT - 1), t);
+  int s = 0;
+  for (int t = 0; t < KT - (NS - 1); ++t) {
+    rg_wait_barrier<(NS - 2) * (LA + LW)>();
+    issue(t + NS - 1, s == 0 ? NS - 1 : s - 1);
+    compute(s);
+    s = s + 1 == NS ? 0 : s + 1;
+  }
+  rg_static_for<0, NS - 1>([&](auto tc) __attribute__((always_inline)) {
+    rg_wait_barrier<(NS - 2 - decltype(tc)::value) * (LA + LW)>();
+    if (decltype(tc)::value < KT) compute(s);
+    s = s + 1 == NS ? 0 : s + 1;
+  });
+}
+
 // WR x WC waves.  gm: tile rows per group of the tile order.
 template <int EPI, int BM, int BN, int NS, int WR, int WC>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_ring(
@@ -81,8 +188,6 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
   constexpr int NW = WR * WC, TH = 64 * NW;
   constexpr int WM = BM / WR, MT = WM / 16;
   constexpr int WN = BN / WC, NT = WN / 16;
-  constexpr int LA = BM / 8 / NW, LW = BN / 8 / NW;   // 1 KB loads per wave per K tile
-  constexpr int SB = (BM + BN) * RG_RB;               // bytes of a stage
   constexpr int CPR = BN / 8, NCH = BM * CPR / TH, CP = BN + 8;
   constexpr bool RES = EPI == EPI_RESID_ATTN || EPI == EPI_RESID_MLP;
   // the residual operands: loaded first where the tile is small (a few
@@ -121,7 +226,6 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     tm = g * gm + rem - tn * h;
   }
   const int m0 = tm * BM, n0 = tn * BN;
-  const int KT = K / RG_BK;
 
   // chunk q = tid + TH u of the output tile: row q / CPR, columns 8 (q % CPR)
   uint4 xv[RES ? NCH : 1], zv[EPI == EPI_RESID_ATTN ? NCH : 1];
@@ -136,96 +240,10 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
   };
   if constexpr (EARLY) res_load();
 
-  // load u of this wave fills rows 8 (NW u + wv) .. + 7 of the operand's tile
-  // in LDS: lane l row l >> 3, slot l & 7, which holds logical 16-byte chunk
-  // (l & 7) ^ ((row >> 1) & 7) -- conflict-free for the 16-row fragment reads.
-  // Rows past M / N repeat the last one (they feed outputs never stored).
-  const bf16_t* pa[LA];
-  const bf16_t* pw[LW];
-#pragma unroll
-  for (int u = 0; u < LA; ++u) {
-    const int r = 8 * (NW * u + wv) + (lane >> 3);
-    pa[u] = A + (size_t)min(m0 + r, M - 1) * lda + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
-  }
-#pragma unroll
-  for (int u = 0; u < LW; ++u) {
-    const int r = 8 * (NW * u + wv) + (lane >> 3);
-    pw[u] = W + (size_t)min(n0 + r, N - 1) * K + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
-  }
-  // (the builtin's operands have plain types: clang's host pass drops a kernel
-  // in which a type-dependent call of its 16-byte form is instantiated)
-  auto issue = [&](int kt, int s) {
-    unsigned char* st = rg_smem + s * SB;
-#pragma unroll
-    for (int u = 0; u < LA; ++u) {
-      const bf16_t* src = pa[u] + kt * RG_BK;
-      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
-    }
-    st += BM * RG_RB;
-#pragma unroll
-    for (int u = 0; u < LW; ++u) {
-      const bf16_t* src = pw[u] + kt * RG_BK;
-      __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
-    }
-  };
-
+  const int r16 = lane & 15, kg = lane >> 4;
   float ss[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) ss[i] = 0.f;
   rg_floatx4 acc[NT][MT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int i = 0; i < MT; ++i) acc[j][i] = (rg_floatx4){0.f, 0.f, 0.f, 0.f};
-
-  // block (N block j, M block i) of C^T = W A^T: a lane holds four consecutive
-  // columns of one row.  The k steps of 32 run in order, as in every GEMM
-  // here: the same bits whatever the tile.
-  const int r16 = lane & 15, kg = lane >> 4, sw = (r16 >> 1) & 7;
-  const int oa = (wm * WM + r16) * RG_RB, ow = BM * RG_RB + (wn * WN + r16) * RG_RB;
-  const int c0 = (kg ^ sw) << 4, c1 = ((4 + kg) ^ sw) << 4;
-  auto compute = [&](int s) {
-    const unsigned char* st = rg_smem + s * SB;
-    rg_bf16x8 a[2][MT], w[2][NT];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-        w[h][j] = *(const rg_bf16x8*)(st + ow + j * 16 * RG_RB + (h ? c1 : c0));
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-        a[h][i] = *(const rg_bf16x8*)(st + oa + i * 16 * RG_RB + (h ? c1 : c0));
-    }
-    __builtin_amdgcn_sched_barrier(0);   // all reads in flight, then the MFMAs
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[h][j], a[h][i], acc[j][i], 0, 0, 0);
-        if constexpr (RMS) ss[i] = rg_sumsq(a[h][i], ss[i]);
-      }
-  };
-
-  // ring: K tile t in stage t % NS, loaded NS - 1 tiles ahead.  The barrier
-  // that follows the wait for tile t also says that every wave is done with
-  // the stage of tile t - 1, which tile t + NS - 1 then overwrites.  (With
-  // fewer K tiles than that the last one is loaded again, and not used.)
-#pragma unroll
-  for (int t = 0; t < NS - 1; ++t) issue(min(t, KT - 1), t);
-  int s = 0;
-  for (int t = 0; t < KT - (NS - 1); ++t) {
-    rg_wait_barrier<(NS - 2) * (LA + LW)>();
-    issue(t + NS - 1, s == 0 ? NS - 1 : s - 1);
-    compute(s);
-    s = s + 1 == NS ? 0 : s + 1;
-  }
-  rg_static_for<0, NS - 1>([&](auto tc) __attribute__((always_inline)) {
-    rg_wait_barrier<(NS - 2 - decltype(tc)::value) * (LA + LW)>();
-    if (decltype(tc)::value < KT) compute(s);
-    s = s + 1 == NS ? 0 : s + 1;
-  });
+  ring_product<BM, BN, NS, WR, WC, RMS>(A, lda, W, M, N, K, m0, n0, wv, lane, acc, ss);
 
   if constexpr (RMS) {
     // a lane's column of C^T is row r16 of its M blocks, whose squares the four
@@ -348,6 +366,146 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
       }
     }
   }
+}
+
+// ---- Polar Express products ---------------------------------------------------
+//
+// `batch` independent products of whole 128 x 128 tiles (EPI_PE_A, EPI_PE_B,
+// EPI_PE_X), the same ring.  sym (PE_A, PE_B): the output is symmetric, only
+// the tiles on and above the diagonal are computed and each one above it is
+// also stored transposed.  The tiles of one matrix are neighbours in an XCD's
+// range, so its operands (1.2 MB at 768 x 768) stay in that L2.  MuonAdam step
+// over the 155M dict: 3.79 -> 3.18 ms against register-staged 128 x 128 tiles
+// (k_gemm_bat; the 15 products 2.63 -> 2.0 ms), the same bits.
+constexpr int PE_T = 128;
+
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_pe_ring(
+    const bf16_t* A, int lda, long long sA, const bf16_t* W, long long sW, int M, int N, int K,
+    EpiArgs ea, long long sOut, long long sX) {
+  constexpr int CPR = PE_T / 8, NCH = PE_T * CPR / 256, CP = PE_T + 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char rg_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wv >> 1, wn = wv & 1, r16 = lane & 15, kg = lane >> 4;
+  const int nbm = M / PE_T, nbn = N / PE_T;
+  const int per = ea.sym ? nbm * (nbm + 1) / 2 : nbm * nbn;
+  const int total = gridDim.x, q8 = total >> 3, r8 = total & 7, x8 = blockIdx.x & 7;
+  const int t = x8 * q8 + min(x8, r8) + (blockIdx.x >> 3);
+  const int z = t / per;
+  int tm = 0, tn = t - z * per;
+  if (ea.sym) {
+    while (tn >= nbm - tm) tn -= nbm - tm++;
+    tn += tm;
+  } else {
+    tm = tn / nbn;
+    tn -= tm * nbn;
+  }
+  const int m0 = tm * PE_T, n0 = tn * PE_T;
+  bf16_t* out = ea.out + z * sOut;
+  const bf16_t* x = ea.x + z * sX;
+
+  float ss[4];
+  rg_floatx4 acc[4][4];
+  ring_product<PE_T, PE_T, 2, 2, 2, false>(A + z * sA, lda, W + z * sW, M, N, K, m0, n0, wv, lane,
+                                           acc, ss);
+  // chunk q = tid + 256 u of the tile: row q / CPR, columns 8 (q % CPR)
+  uint4 xv[EPI == EPI_PE_A ? 1 : NCH];
+  if constexpr (EPI != EPI_PE_A) {
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int q = tid + 256 * u;
+      xv[u] = *(const uint4*)(x + (size_t)(m0 + q / CPR) * ea.ldr + n0 + (q % CPR) * 8);
+    }
+  }
+  __syncthreads();   // every wave is done with the last K tile
+  bf16_t* tile = (bf16_t*)rg_smem;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const rg_floatx4 y = acc[j][i];
+      *(uint2*)(tile + (wm * 64 + i * 16 + r16) * CP + wn * 64 + j * 16 + 4 * kg) =
+          make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
+    }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NCH; ++u) {
+    const int q = tid + 256 * u, ml = q / CPR, c8 = (q % CPR) * 8;
+    uint4* sy = (uint4*)(tile + ml * CP + c8);
+    uint4 o = *sy;
+    if constexpr (EPI != EPI_PE_A) {
+      // each eager product and sum rounded to bf16
+      const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
+      uint32_t w[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const uint32_t a = pack2(ea.s0 * lo_f(xw[f]), ea.s0 * hi_f(xw[f]));
+        if constexpr (EPI == EPI_PE_B) w[f] = pack2(ea.s1 * lo_f(w[f]), ea.s1 * hi_f(w[f]));
+        w[f] = pack2(lo_f(a) + lo_f(w[f]), hi_f(a) + hi_f(w[f]));
+      }
+      o = make_uint4(w[0], w[1], w[2], w[3]);
+      *sy = o;   // kept for a transposed copy
+    }
+    *(uint4*)(out + (size_t)(m0 + ml) * ea.ldo + n0 + c8) = o;
+  }
+  // transposed: PE_X's copy x'^T, or the mirror of a tile above the diagonal
+  bf16_t* dst = EPI == EPI_PE_X ? (ea.outT ? ea.outT + z * sOut : nullptr)
+                                : (ea.sym && tn != tm ? out : nullptr);
+  if (!dst) return;
+  const int ld = EPI == EPI_PE_X ? ea.ldoT : ea.ldo;
+  if constexpr (EPI != EPI_PE_A) __syncthreads();
+  // a thread takes a column pair and 32 rows, 16-byte runs of each column
+  const int cp = tid & 63, rb = tid >> 6;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int r0 = rb * 32 + 8 * g;
+    uint32_t w[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = *(const uint32_t*)(tile + (r0 + e) * CP + 2 * cp);
+    uint4 c0, c1;
+    c0.x = (w[0] & 0xffffu) | (w[1] << 16); c0.y = (w[2] & 0xffffu) | (w[3] << 16);
+    c0.z = (w[4] & 0xffffu) | (w[5] << 16); c0.w = (w[6] & 0xffffu) | (w[7] << 16);
+    c1.x = (w[0] >> 16) | (w[1] & 0xffff0000u); c1.y = (w[2] >> 16) | (w[3] & 0xffff0000u);
+    c1.z = (w[4] >> 16) | (w[5] & 0xffff0000u); c1.w = (w[6] >> 16) | (w[7] & 0xffff0000u);
+    bf16_t* d = dst + (size_t)(n0 + 2 * cp) * ld + m0 + r0;
+    *(uint4*)d = c0;
+    *(uint4*)(d + ld) = c1;
+  }
+}
+
+// Whole tiles, 16-byte rows, a square output where it is symmetric.
+bool pe_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                  const EpiArgs& ea, long long sA, long long sW, long long sOut, long long sX,
+                  int batch) {
+  if (M % PE_T || N % PE_T || K % RG_BK || K < RG_BK || M < PE_T || N < PE_T) return false;
+  if ((long long)(M / PE_T) * (N / PE_T) * batch > (1 << 30)) return false;
+  if ((lda | ea.ldo) % 8 || ((sA | sW | sOut) & 7) ||
+      (((uintptr_t)A | (uintptr_t)W | (uintptr_t)ea.out) & 15))
+    return false;
+  if (epi != EPI_PE_A && (ea.ldr % 8 || (sX & 7) || ((uintptr_t)ea.x & 15))) return false;
+  if (epi == EPI_PE_X && ea.outT && (ea.ldoT % 8 || ((uintptr_t)ea.outT & 15))) return false;
+  return epi == EPI_PE_X ? !ea.sym : (!ea.sym || M == N);
+}
+
+hipError_t pe_ring(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W, long long sW,
+                   int M, int N, int K, const EpiArgs& ea, long long sOut, long long sX, int batch,
+                   hipStream_t st) {
+  const int nbm = M / PE_T, nbn = N / PE_T;
+  const dim3 grid((ea.sym ? nbm * (nbm + 1) / 2 : nbm * nbn) * batch);
+  constexpr size_t lds = rg_lds_bytes<PE_T, PE_T, 2>();   // 64 KB
+#define PE_CASE(E)                                                                              \
+  case E:                                                                                       \
+    hipLaunchKernelGGL((k_pe_ring<E>), grid, dim3(256), lds, st, A, lda, sA, W, sW, M, N, K, ea, \
+                       sOut, sX);                                                               \
+    return hipGetLastError();
+  switch (epi) {
+    PE_CASE(EPI_PE_A)
+    PE_CASE(EPI_PE_B)
+    PE_CASE(EPI_PE_X)
+  }
+#undef PE_CASE
+  return hipErrorInvalidValue;
 }
 
 namespace {

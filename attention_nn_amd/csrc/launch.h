@@ -28,12 +28,13 @@ namespace ann {
 //                   largest first (0 past the valid columns), and its 9th
 //                   largest word to cand_r[m nt + t]; softcap(z) -> logits fp32
 //                   (if set).  No z is stored (sample.py:44-49 via sample_cand)
+//   EPI_PE_A        (Polar Express) out = bf16(y)                               (muon.py:36)
 //   EPI_PE_B        (Polar Express) out = bf16(bf16(s0*x) + bf16(s1*bf16(y)))  (muon.py:37)
 //   EPI_PE_X        (Polar Express) out = bf16(bf16(s0*x) + bf16(y))           (muon.py:38,42)
 //                   x is the epilogue's second operand (M, ldr); when outT is set
 //                   the same values also go to outT (N, ldoT), transposed
 enum { EPI_STORE = 0, EPI_RELU2 = 1, EPI_RESID_ATTN = 2, EPI_RESID_MLP = 3, EPI_LOGITS = 4,
-       EPI_QKV = 5, EPI_CE = 6, EPI_PE_B = 7, EPI_PE_X = 8, EPI_TOPK = 9 };
+       EPI_QKV = 5, EPI_CE = 6, EPI_PE_B = 7, EPI_PE_X = 8, EPI_TOPK = 9, EPI_PE_A = 10 };
 
 // Candidates a 128-column lm_head tile emits per row (EPI_TOPK).
 constexpr int TK_M = 8;
@@ -76,7 +77,7 @@ struct EpiArgs {
   // PE_X: transposed copy of the output, or null
   bf16_t* outT;
   int ldoT;
-  // batched STORE / PE_B with a symmetric M x M output (x x^T, b A + c A A):
+  // PE_A / PE_B with a symmetric M x M output (x x^T, b A + c A A):
   // only the tiles on and above the diagonal are computed, each one above it
   // also stored transposed at the mirrored position
   int sym;
@@ -118,8 +119,6 @@ hipError_t argmax_finalize(const unsigned long long* keys, int nkeys, int M, int
 // rms: A rows RMS-normalised in the kernel (K <= 3072).
 bool gemm_skinny_fits(int M, int N, int K, bool rms);
 bool gemm_qkv_fits(int M, int N, int K, const EpiArgs& ea);
-// k_gemm over `batch` independent problems (blockIdx.z); epilogues STORE,
-// PE_B, PE_X; sOut / sX are the batch strides of ea.out / ea.x.
 // Projections of the prefill, the training forward and whole-context logits:
 // 32 x 64 .. 128 x 192 tiles by shape, K tiles streamed into an LDS ring
 // (gemm_ring.hip).  y = a @ W^T; where gemm_ring_rms says so (EPI_STORE,
@@ -146,6 +145,15 @@ hipError_t gemm_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int
                     const EpiArgs& ea, hipStream_t st);
 // Compute units of the current device (256 where the query fails).
 int device_cus();
+// `batch` independent products (sA, sW, sOut, sX: strides of A, W, ea.out /
+// ea.outT, ea.x); epilogues PE_A, PE_B, PE_X.  pe_ring (gemm_ring.hip) where
+// whole 128 x 128 tiles fit, else k_gemm_bat.
+bool pe_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
+                  const EpiArgs& ea, long long sA, long long sW, long long sOut, long long sX,
+                  int batch);
+hipError_t pe_ring(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W, long long sW,
+                   int M, int N, int K, const EpiArgs& ea, long long sOut, long long sX, int batch,
+                   hipStream_t st);
 hipError_t gemm_batched(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W,
                         long long sW, int M, int N, int K, const EpiArgs& ea, long long sOut,
                         long long sX, int batch, hipStream_t st);

@@ -548,10 +548,8 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   static_assert(EPI != EPI_TOPK || BN % 128 == 0, "whole 128-column candidate tiles");
   // staged epilogues (TOPK; PE_B / PE_X on full tiles) reuse the LDS for a bf16
   // BM x BN tile of row pitch BN + 8
-  // the batched plain store stages its 128 x 128 tiles for the symmetric form
-  constexpr bool STAGE_STORE = EPI == EPI_STORE && BM == GM_BM && BN == GM_BN && DEPTH == 1;
   constexpr bool STAGED =
-      EPI == EPI_PE_B || EPI == EPI_PE_X || EPI == EPI_TOPK || STAGE_STORE;
+      EPI == EPI_PE_B || EPI == EPI_PE_X || EPI == EPI_TOPK;
   constexpr int SMEM = (BM + BN) * GM_BK > (STAGED ? BM * (BN + 8) : 0)
                            ? (BM + BN) * GM_BK
                            : BM * (BN + 8);
@@ -567,17 +565,7 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   // grid (correct under any dispatch order); batched launches keep the
   // identity.  Measured 3-6% faster per prefill GEMM.
   int tm = blockIdx.y, tn = blockIdx.x;
-  if (ea.sym) {
-    // symmetric output: blockIdx.x walks the tiles tn >= tm row by row
-    const int nb = (M + BM - 1) / BM;
-    int t = blockIdx.x;
-    tm = 0;
-    while (t >= nb - tm) {
-      t -= nb - tm;
-      ++tm;
-    }
-    tn = tm + t;
-  } else if (gridDim.z == 1) {
+  if (gridDim.z == 1) {
     const int nbn = gridDim.x, total = nbn * gridDim.y;
     const int bid = blockIdx.y * nbn + blockIdx.x;
     const int x = bid & 7, q = total >> 3, r = total & 7;
@@ -716,31 +704,6 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   };
   if constexpr (!SWAP) {
     // C layout of the 16x16 MFMA: lane holds column (lane & 15), rows 4 (lane >> 4) + r
-    if constexpr (STAGE_STORE) {
-      // symmetric form (full tiles, host-checked): staged bf16 tile, 16-byte
-      // row chunks, and the mirrored tile^T above the diagonal
-      if (ea.sym) {
-        constexpr int CP = BN + 8, CPR = BN / 8, NCH = BM * CPR / 256;
-        __syncthreads();   // every wave is done with the last K tile in LDS
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              smem[(wm * WM + i * 16 + (lane >> 4) * 4 + r) * CP + wn * WN + j * 16 + r16] =
-                  f2bf(acc[j][i][r]);
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < NCH; ++u) {
-          const int q = tid + 256 * u, ml = q / CPR, c8 = (q % CPR) * 8;
-          *(uint4*)(ea.out + (size_t)(m0 + ml) * ea.ldo + n0 + c8) =
-              *(const uint4*)(smem + ml * CP + c8);
-        }
-        if (tn != tm) store_transposed(ea.out, ea.ldo, std::integral_constant<int, CP>{});
-        return;
-      }
-    }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -866,20 +829,10 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
           *(uint4*)(ea.out + (size_t)(m0 + ml) * ea.ldo + n0 + c8) = ov;
           *sy = ov;   // kept for a transposed copy
         }
-        // PE_X: the transposed copy x'^T; PE_B in the symmetric form: the
-        // mirrored tile above the diagonal
-        bf16_t* tdst = nullptr;
-        int tld = 0;
-        if constexpr (EPI == EPI_PE_X) {
-          tdst = ea.outT;
-          tld = ea.ldoT;
-        } else if (ea.sym && tn != tm) {
-          tdst = ea.out;
-          tld = ea.ldo;
-        }
-        if (tdst) {
+        // PE_X: the transposed copy x'^T
+        if (EPI == EPI_PE_X && ea.outT) {
           __syncthreads();
-          store_transposed(tdst, tld, std::integral_constant<int, CP>{});
+          store_transposed(ea.outT, ea.ldoT, std::integral_constant<int, CP>{});
         }
         return;
       }
@@ -1274,28 +1227,21 @@ hipError_t gemm_batched(int epi, const bf16_t* A, int lda, long long sA, const b
                         long long sX, int batch, hipStream_t st) {
   if (K % GM_BK != 0 || M <= 0 || N <= 0 || batch <= 0 || batch > 65535)
     return hipErrorInvalidValue;
+  // batches of whole 128 x 128 tiles: the ring
+  if (pe_ring_fits(epi, A, lda, W, M, N, K, ea, sA, sW, sOut, sX, batch))
+    return pe_ring(epi, A, lda, sA, W, sW, M, N, K, ea, sOut, sX, batch, st);
   const int bm = M <= 64 ? 64 : GM_BM;
   dim3 grid((N + GM_BN - 1) / GM_BN, (M + bm - 1) / bm, batch);
-  EpiArgs e2 = ea;
-  // symmetric form: square outputs of whole 128 x 128 tiles, 16-byte aligned
-  e2.sym = ea.sym && (epi == EPI_STORE || epi == EPI_PE_B) && M == N && bm == GM_BM &&
-           M % GM_BM == 0 && ea.ldo % 8 == 0 && ((uintptr_t)ea.out & 15) == 0 &&
-           sOut % 8 == 0 && (epi != EPI_PE_B || (ea.ldr % 8 == 0 && sX % 8 == 0 &&
-                                                 ((uintptr_t)ea.x & 15) == 0));
-  if (e2.sym) {
-    const int nb = M / GM_BM;
-    grid = dim3(nb * (nb + 1) / 2, 1, batch);
-  }
 #define ANN_GB(E)                                                                              \
   if (bm == 64)                                                                                \
     hipLaunchKernelGGL((k_gemm_bat<E, 64>), grid, dim3(256), 0, st, A, lda, sA, W, sW, M, N,   \
-                       K, e2, sOut, sX);                                                       \
+                       K, ea, sOut, sX);                                                       \
   else                                                                                         \
     hipLaunchKernelGGL((k_gemm_bat<E, GM_BM>), grid, dim3(256), 0, st, A, lda, sA, W, sW, M,   \
-                       N, K, e2, sOut, sX);                                                    \
+                       N, K, ea, sOut, sX);                                                    \
   break;
   switch (epi) {
-    case EPI_STORE: ANN_GB(EPI_STORE)
+    case EPI_PE_A: ANN_GB(EPI_STORE)
     case EPI_PE_B: ANN_GB(EPI_PE_B)
     case EPI_PE_X: ANN_GB(EPI_PE_X)
     default: return hipErrorInvalidValue;

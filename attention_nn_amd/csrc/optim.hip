@@ -231,7 +231,7 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       ea.out = am;
       ea.ldo = M;
       ea.sym = 1;
-      e = gemm_batched(EPI_STORE, cur, N, (long long)mn, cur, (long long)mn, M, M, N, ea,
+      e = gemm_batched(EPI_PE_A, cur, N, (long long)mn, cur, (long long)mn, M, M, N, ea,
                        (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
       // B = b A + c (A A)
@@ -260,7 +260,7 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       ea.out = am;
       ea.ldo = N;
       ea.sym = 1;
-      e = gemm_batched(EPI_STORE, xt, M, (long long)mn, xt, (long long)mn, N, N, M, ea,
+      e = gemm_batched(EPI_PE_A, xt, M, (long long)mn, xt, (long long)mn, N, N, M, ea,
                        (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
       ea.out = bm;
