@@ -907,16 +907,16 @@ __global__ __launch_bounds__(256) void k_gemm_sk(const bf16_t* __restrict__ A, i
 
 // ---- skinny MFMA GEMM, LDS-staged (decode, M <= 128, no RMS prologue) ------
 //
-// Same work split as k_gemm_sk (one 16T x 16T tile per work-group, the four
-// waves split K into quarters), but each wave brings its quarter of the A and
+// Same work split as k_gemm_sk (one 16T x 16T tile per work-group, the NV
+// waves split K evenly), but each wave brings its part of the A and
 // W tiles in with contiguous 16-byte loads -- lanes along a row, not the
 // 16-row x 64-byte MFMA fragment pattern, which moves ~3x fewer bytes per CU
 // cycle -- into its own padded LDS region, in rounds of KC k-steps, and reads
 // the fragments back with ds_read_b128.  A wave touches only its own region,
 // so no barrier is needed until the cross-wave sum, whose partials go into
 // each wave's own (then finished) region.  Operands are swapped for the
-// read-modify-write epilogues (8-byte accesses), as in k_gemm.  Bit-identical
-// to k_gemm_sk (same k order per wave, same wave order).
+// read-modify-write epilogues (8-byte accesses), as in k_gemm.  With
+// four waves bit-identical to k_gemm_sk (same k order per wave, same wave order).
 // RMS: the rows of A are normalised in the kernel (model.py:48-49 with the
 // bf16 output of an eager op): before the first round each wave reads its K
 // quarter of the tile's A rows with contiguous loads, leaves per-chunk sums of
@@ -926,8 +926,8 @@ __global__ __launch_bounds__(256) void k_gemm_sk(const bf16_t* __restrict__ A, i
 // D: rounds in flight per wave (a register ring): round r + D is loaded as
 // soon as round r is in LDS, so a wave waits on memory about once per D
 // rounds instead of once per round.
-template <int EPI, bool RMS, int KC, int T, int D>
-__global__ __launch_bounds__(256) void k_gemm_sk2(const bf16_t* __restrict__ A, int lda,
+template <int EPI, bool RMS, int KC, int T, int D, int NV = 4>
+__global__ __launch_bounds__(64 * NV) void k_gemm_sk2(const bf16_t* __restrict__ A, int lda,
                                                   const bf16_t* __restrict__ W, int M, int N,
                                                   int K, float eps, EpiArgs ea) {
   constexpr int R = 16 * T;        // rows per operand tile
@@ -937,11 +937,11 @@ __global__ __launch_bounds__(256) void k_gemm_sk2(const bf16_t* __restrict__ A, 
   constexpr int REGION = 2 * R * PITCH;
   static_assert(REGION * 16 >= T * T * 64 * 16, "partials fit a wave's region");
   constexpr bool SWAP = EPI != EPI_STORE && EPI != EPI_RELU2;
-  __shared__ uint4 s_t[4][REGION];
-  __shared__ float s_ss[RMS ? 4 : 1][R];
+  __shared__ uint4 s_t[NV][REGION];
+  __shared__ float s_ss[RMS ? NV : 1][R];
   const int tid = threadIdx.x, lane = tid & 63, wk = tid >> 6;
   const int n0 = blockIdx.x * 16 * T, m0 = blockIdx.y * 16 * T;
-  const int kw = K >> 7;            // k-steps of 32 per wave
+  const int kw = K / (32 * NV);            // k-steps of 32 per wave
   const int kbase = wk * kw * 32;   // first k of this wave's quarter
   uint4* sa = s_t[wk];
   uint4* sw = s_t[wk] + R * PITCH;
@@ -989,7 +989,9 @@ __global__ __launch_bounds__(256) void k_gemm_sk2(const bf16_t* __restrict__ A, 
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       const int r = 16 * t + r16;
-      const float tt = ((s_ss[0][r] + s_ss[1][r]) + s_ss[2][r]) + s_ss[3][r];
+      float tt = s_ss[0][r];
+#pragma unroll
+      for (int j = 1; j < NV; ++j) tt += s_ss[j][r];
       scale[t] = rsqrtf(tt / (float)K + eps);
     }
     __builtin_amdgcn_wave_barrier();
@@ -1077,7 +1079,7 @@ __global__ __launch_bounds__(256) void k_gemm_sk2(const bf16_t* __restrict__ A, 
     __builtin_amdgcn_wave_barrier();
     asm volatile("" ::: "memory");
   });
-  // partials of waves 1..3 into their own regions, summed by wave 0 in order
+  // partials of waves 1 .. NV - 1 into their own regions, summed by wave 0 in order
   floatx4_t* red = (floatx4_t*)s_t[wk];
   if (wk > 0) {
 #pragma unroll
@@ -1094,7 +1096,7 @@ __global__ __launch_bounds__(256) void k_gemm_sk2(const bf16_t* __restrict__ A, 
     for (int tw = 0; tw < T; ++tw) {
       floatx4_t v = acc[ta][tw];
 #pragma unroll
-      for (int j = 1; j < 4; ++j) {
+      for (int j = 1; j < NV; ++j) {
         const floatx4_t p = ((const floatx4_t*)s_t[j])[(ta * T + tw) * 64 + lane];
         v[0] += p[0];
         v[1] += p[1];
@@ -1151,6 +1153,35 @@ hipError_t gemm_skinny(int epi, bool rms, const bf16_t* A, int lda, const bf16_t
     // flight per wave (cfg5 decode 3421 -> 3310 us per step, measured); the
     // 16 x 16 tiles measured ~1% slower with it (batch-64 proj: 3 rounds)
     const int xd = T == 2 && kw % 4 == 0 && (kw / 4) % 3 == 0 ? 3 : 1;
+    // The o / proj projections on 16 x 16 tiles: eight waves instead of four
+    // halve each wave's chain of rounds where their larger LDS costs no
+    // resident work-group: short chains (K <= 768: 51 KB), or at most one work-
+    // group per CU (102 KB).  155M decode step of 7 / 16 / 64 / 80 rows 322 ->
+    // 310, 337 -> 325, 470 -> 459, 552 -> 540 us, d 1536 at 8 rows (three
+    // layers) 179 -> 169; proj with more work-groups than CUs is slower (100
+    // rows 596 -> 615).  16 waves: within 1% of eight.
+    static const int cus = device_cus();
+    const int kw8 = K / 256;
+    if ((epi == EPI_RESID_ATTN || epi == EPI_RESID_MLP) && T == 1 && K % 256 == 0 &&
+        (kw8 <= 3 || (int)(grid.x * grid.y) <= cus)) {
+#define ANN_SK2_W8(E)                                                                            \
+  if (kw8 <= 3)                                                                                  \
+    hipLaunchKernelGGL((k_gemm_sk2<E, false, 3, 1, 1, 8>), grid, dim3(512), 0, st, A, lda, W, M,  \
+                       N, K, eps, ea);                                                           \
+  else if (kw8 % 6 == 0)                                                                         \
+    hipLaunchKernelGGL((k_gemm_sk2<E, false, 6, 1, 1, 8>), grid, dim3(512), 0, st, A, lda, W, M,  \
+                       N, K, eps, ea);                                                           \
+  else                                                                                           \
+    hipLaunchKernelGGL((k_gemm_sk2<E, false, 4, 1, 1, 8>), grid, dim3(512), 0, st, A, lda, W, M,  \
+                       N, K, eps, ea);
+      if (epi == EPI_RESID_ATTN) {
+        ANN_SK2_W8(EPI_RESID_ATTN)
+      } else {
+        ANN_SK2_W8(EPI_RESID_MLP)
+      }
+#undef ANN_SK2_W8
+      return hipGetLastError();
+    }
 #define ANN_SK2_R(E, R)                                                                          \
   if (T == 1) {                                                                                  \
     if (kw <= 6)                                                                                 \
