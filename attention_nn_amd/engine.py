@@ -11,6 +11,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from ._stream import current_stream
 from .config import V_SAMPLE
 from .weights import check_params
 
@@ -20,10 +21,6 @@ PARAM_ORDER = ("embed", "lm_head", "attn_bank", "fc_bank", "proj_bank",
 
 def _ptr(t):
     return ctypes.c_void_p(t.data_ptr())
-
-
-def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 class Engine:
@@ -66,7 +63,7 @@ class Engine:
                for k in PARAM_ORDER}
         p = _lib.AnnParamsF32(**{k: src[k].data_ptr() for k in PARAM_ORDER})
         _lib.check(_lib.lib().ann_pack_weights(self._ctx, ctypes.byref(p), _ptr(self.wbuf),
-                                               self.wbuf.numel(), _stream()))
+                                               self.wbuf.numel(), current_stream()))
         torch.cuda.current_stream().synchronize()
         del src
 
@@ -115,7 +112,7 @@ class Engine:
     def check_device(self):
         """Raise if a bounded cross-work-group wait of the persistent decode
         step timed out since the last check (synchronises the stream)."""
-        _lib.check(_lib.lib().ann_check_device(self._ctx, _stream()))
+        _lib.check(_lib.lib().ann_check_device(self._ctx, current_stream()))
 
     def reset(self):
         _lib.check(_lib.lib().ann_reset(self._ctx))
@@ -127,7 +124,7 @@ class Engine:
         t = self._tokens(tokens, 2)
         B, T = t.shape
         out = torch.empty((B, T, self.cfg.vocab_size), dtype=torch.float32, device=self.device)
-        _lib.check(_lib.lib().ann_forward_logits(self._ctx, _ptr(t), B, T, _ptr(out), _stream()))
+        _lib.check(_lib.lib().ann_forward_logits(self._ctx, _ptr(t), B, T, _ptr(out), current_stream()))
         self.batch = B
         return out
 
@@ -143,7 +140,7 @@ class Engine:
         mean = torch.empty((), dtype=torch.float32, device=self.device)
         per = torch.empty((B * T,), dtype=torch.float32, device=self.device) if rows else None
         _lib.check(_lib.lib().ann_forward_loss(self._ctx, _ptr(t), _ptr(g), B, T, _ptr(mean),
-                                               _ptr(per) if rows else None, _stream()))
+                                               _ptr(per) if rows else None, current_stream()))
         self.batch = B
         return (mean, per) if rows else mean
 
@@ -156,7 +153,7 @@ class Engine:
             if want_logits else None
         s = self._sampling(temperature, top_k, seed, step)
         _lib.check(_lib.lib().ann_prefill(self._ctx, _ptr(t), B, T, ctypes.byref(s), _ptr(nxt),
-                                          _ptr(lg) if lg is not None else None, _stream()))
+                                          _ptr(lg) if lg is not None else None, current_stream()))
         self.batch = B
         return nxt, lg
 
@@ -170,5 +167,5 @@ class Engine:
             if want_logits else None
         s = self._sampling(temperature, top_k, seed, step)
         _lib.check(_lib.lib().ann_decode_step(self._ctx, _ptr(t), B, ctypes.byref(s), _ptr(nxt),
-                                              _ptr(lg) if lg is not None else None, _stream()))
+                                              _ptr(lg) if lg is not None else None, current_stream()))
         return nxt, lg

@@ -16,6 +16,7 @@ import ctypes
 import torch
 
 from . import _lib
+from ._stream import current_stream
 
 
 def _dt(x):
@@ -32,10 +33,6 @@ def _gpu(x):
     return x.contiguous()
 
 
-def _s():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
 def _p(t):
     return ctypes.c_void_p(t.data_ptr())
 
@@ -43,7 +40,7 @@ def _p(t):
 def relu2(x):
     x = _gpu(x)
     y = torch.empty_like(x)
-    _lib.check(_lib.lib().ann_op_relu2(_p(x), _p(y), x.numel(), _dt(x), _s()))
+    _lib.check(_lib.lib().ann_op_relu2(_p(x), _p(y), x.numel(), _dt(x), current_stream()))
     return y
 
 
@@ -57,14 +54,14 @@ def rope_ht(x, cs, sn, pos0=0, inverse=False):
         raise ValueError("tables must be (>= pos0 + T, D/4)")
     y = torch.empty_like(x)
     _lib.check(_lib.lib().ann_op_rope_ht(_p(x), _p(y), _p(cs), _p(sn), B, T, H, D, pos0,
-                                         int(bool(inverse)), _dt(x), _s()))
+                                         int(bool(inverse)), _dt(x), current_stream()))
     return y
 
 
 def make_rope_tables(seq_len, head_dim, base=1024.0, device="cuda"):
     cs = torch.empty((seq_len, head_dim // 4), dtype=torch.float32, device=device)
     sn = torch.empty_like(cs)
-    _lib.check(_lib.lib().ann_op_rope_tables(_p(cs), _p(sn), seq_len, head_dim, float(base), _s()))
+    _lib.check(_lib.lib().ann_op_rope_tables(_p(cs), _p(sn), seq_len, head_dim, float(base), current_stream()))
     return cs, sn
 
 
@@ -73,5 +70,5 @@ def rms(x, eps=1e-6):
     y = torch.empty_like(x)
     dim = x.shape[-1]
     _lib.check(_lib.lib().ann_op_rms_norm(_p(x), _p(y), x.numel() // dim, dim, float(eps),
-                                          _dt(x), _s()))
+                                          _dt(x), current_stream()))
     return y
