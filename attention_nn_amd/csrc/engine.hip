@@ -1176,6 +1176,22 @@ int ann_op_normuon(const void* v, float* second_mom, int32_t batch, int32_t M, i
   return ANN_OK;
 }
 
+int ann_op_normuon_update(const void* v, float* second_mom, int32_t batch, int32_t M, int32_t N,
+                          float beta2, const float* p, float lr, float wd, float* p_out, void* ws,
+                          size_t ws_bytes, void* stream) {
+  if (!v || !second_mom || !p || !p_out || !ws) return fail(ANN_E_ARG, "null argument");
+  if (batch <= 0 || batch > 65535 || M <= 0 || N <= 0 || N % 8 ||
+      (long long)M * N >= (1LL << 33))
+    return fail(ANN_E_ARG, "bad shape batch=%d M=%d N=%d (N a multiple of 8)", batch, M, N);
+  if (((uintptr_t)v | (uintptr_t)p | (uintptr_t)p_out) & 15)
+    return fail(ANN_E_ARG, "v, p and p_out must be 16-byte aligned");
+  if (ws_bytes < normuon_ws_bytes(batch, M, N))
+    return fail(ANN_E_ARG, "workspace %zu < %zu bytes", ws_bytes, normuon_ws_bytes(batch, M, N));
+  HIPCHK(normuon_update((const bf16_t*)v, second_mom, batch, M, N, beta2, p, lr, wd, p_out, ws,
+                        ws_bytes, (hipStream_t)stream));
+  return ANN_OK;
+}
+
 size_t ann_op_normuon_noalloc_max_bytes(void) { return NM_SCRATCH_BYTES; }
 
 int ann_op_normuon_noalloc(const void* v, float* second_mom, int32_t batch, int32_t M, int32_t N,

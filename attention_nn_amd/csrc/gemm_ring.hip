@@ -34,6 +34,9 @@ typedef float rg_floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t rg_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 rg_bf16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void rg_lds_void;
+typedef short rg_v4i16 __attribute__((ext_vector_type(4)));
+typedef short rg_v8i16 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) rg_v4i16 rg_lds_v4i16;
 
 // c + the sum of squares of a fragment's eight values (v_dot2_f32_bf16)
 __device__ __forceinline__ float rg_sumsq(const rg_bf16x8& a, float c) {
@@ -76,13 +79,15 @@ constexpr size_t rg_lds_bytes() {
 // acc = the (m0, n0) tile of C^T = W A^T: block (N block j, M block i), so that a
 // lane holds four consecutive columns of one row; ss (SQ): this lane's part of
 // the sums of squares of the A rows (row r16 of M block i, summed over the
-// four lanes of that r16).  W is (N, K).  LDS from rg_smem's start; a barrier
-// has to follow before it is written again.
-template <int BM, int BN, int NS, int WR, int WC, bool SQ>
+// four lanes of that r16).  W is (N, K); WT: (K, N), rows of ldw values, whose
+// fragments come out of LDS through the transposing read.  LDS from rg_smem's
+// start; a barrier has to follow before it is written again.
+template <int BM, int BN, int NS, int WR, int WC, bool SQ, bool WT = false>
 __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf16_t* W, int M,
                                              int N, int K, int m0, int n0, int wv, int lane,
                                              rg_floatx4 (&acc)[BN / WC / 16][BM / WR / 16],
-                                             float (&ss)[BM / WR / 16]) {
+                                             float (&ss)[BM / WR / 16], int ldw = 0) {
+  static_assert(!WT || (BN == 128 && WR * WC == 4 && NS == 2), "256-byte rows of a K tile");
   constexpr int NW = WR * WC;
   constexpr int WM = BM / WR, MT = WM / 16;
   constexpr int WN = BN / WC, NT = WN / 16;
@@ -103,9 +108,19 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
   }
 #pragma unroll
   for (int u = 0; u < LW; ++u) {
-    const int r = 8 * (NW * u + wv) + (lane >> 3);
-    pw[u] = W + (size_t)min(n0 + r, N - 1) * K + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+    if constexpr (WT) {
+      // four K rows of 256 bytes a load: row lane >> 4, slot lane & 15 holding
+      // chunk slot ^ 2 s(row), s = row bits 0, 1 and 3: the transposing reads of
+      // a half wave (8 rows, two chunks each) meet every bank group once
+      const int r = 4 * (NW * u + wv) + (lane >> 4);
+      const int c = (lane & 15) ^ (2 * ((r & 3) | ((r >> 1) & 4)));
+      pw[u] = W + (size_t)r * ldw + n0 + c * 8;
+    } else {
+      const int r = 8 * (NW * u + wv) + (lane >> 3);
+      pw[u] = W + (size_t)min(n0 + r, N - 1) * K + (((lane & 7) ^ ((r >> 1) & 7)) << 3);
+    }
   }
+  const size_t wstep = WT ? (size_t)RG_BK * ldw : (size_t)RG_BK;
   // (the builtin's operands have plain types: clang's host pass drops a kernel
   // in which a type-dependent call of its 16-byte form is instantiated)
   auto issue = [&](int kt, int s) {
@@ -118,7 +133,7 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
     st += BM * RG_RB;
 #pragma unroll
     for (int u = 0; u < LW; ++u) {
-      const bf16_t* src = pw[u] + kt * RG_BK;
+      const bf16_t* src = pw[u] + kt * wstep;
       __builtin_amdgcn_global_load_lds(src, (rg_lds_void*)(st + (NW * u + wv) * 1024), 16, 0, 0);
     }
   };
@@ -136,18 +151,37 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
   const int wm = wv / WC, wn = wv % WC;
   const int oa = (wm * WM + r16) * RG_RB, ow = BM * RG_RB + (wn * WN + r16) * RG_RB;
   const int c0 = (kg ^ sw) << 4, c1 = ((4 + kg) ^ sw) << 4;
-  auto compute = [&](int s) {
+  // WT: within each 16-lane group, lane m receives column m of four K rows, row
+  // e of them addressed by lanes 4e .. 4e + 3; k = 8 kg + 0 .. 3 and + 4 .. 7 in
+  // two reads give the fragment of the untransposed form
+  int tw[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    tw[j] = BM * RG_RB + (8 * kg + (r16 >> 2)) * 256 +
+            ((((wn * WN + j * 16) / 8) ^ (2 * ((r16 >> 2) | ((kg & 1) << 2)))) +
+             ((r16 & 3) >> 1)) * 16 + (r16 & 1) * 8;
+  auto compute = [&](int s, auto&& mid) {
     const unsigned char* st = rg_smem + s * SB;
     rg_bf16x8 a[2][MT], w[2][NT];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-        w[h][j] = *(const rg_bf16x8*)(st + ow + j * 16 * RG_RB + (h ? c1 : c0));
+      for (int j = 0; j < NT; ++j) {
+        if constexpr (WT) {
+          const unsigned char* src = st + tw[j] + h * 32 * 256;
+          const rg_v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rg_lds_v4i16*)src);
+          const rg_v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((rg_lds_v4i16*)(src + 4 * 256));
+          const rg_v8i16 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          w[h][j] = __builtin_bit_cast(rg_bf16x8, v);
+        } else {
+          w[h][j] = *(const rg_bf16x8*)(st + ow + j * 16 * RG_RB + (h ? c1 : c0));
+        }
+      }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         a[h][i] = *(const rg_bf16x8*)(st + oa + i * 16 * RG_RB + (h ? c1 : c0));
     }
+    mid();
     __builtin_amdgcn_sched_barrier(0);   // all reads in flight, then the MFMAs
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -169,13 +203,18 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
   int s = 0;
   for (int t = 0; t < KT - (NS - 1); ++t) {
     rg_wait_barrier<(NS - 2) * (LA + LW)>();
-    issue(t + NS - 1, s == 0 ? NS - 1 : s - 1);
-    compute(s);
+    // WT: the loads go out after the LDS reads, before whose transposing form
+    // the compiler waits for every load into LDS in flight
+    auto next = [&]() { issue(t + NS - 1, s == 0 ? NS - 1 : s - 1); };
+    if constexpr (!WT) next();
+    compute(s, [&]() {
+      if constexpr (WT) next();
+    });
     s = s + 1 == NS ? 0 : s + 1;
   }
   rg_static_for<0, NS - 1>([&](auto tc) __attribute__((always_inline)) {
     rg_wait_barrier<(NS - 2 - decltype(tc)::value) * (LA + LW)>();
-    if (decltype(tc)::value < KT) compute(s);
+    if (decltype(tc)::value < KT) compute(s, []() {});
     s = s + 1 == NS ? 0 : s + 1;
   });
 }
@@ -377,6 +416,9 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
 // range, so its operands (1.2 MB at 768 x 768) stay in that L2.  MuonAdam step
 // over the 155M dict: 3.79 -> 3.18 ms against register-staged 128 x 128 tiles
 // (k_gemm_bat; the 15 products 2.63 -> 2.0 ms), the same bits.
+// PE_X (x' = a x + B x) reads x as the (K, N) operand it is: 60 us a 155M bank
+// against 71 with a transposed copy written by each epilogue and read by the
+// next product.
 constexpr int PE_T = 128;
 
 template <int EPI>
@@ -407,8 +449,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
   float ss[4];
   rg_floatx4 acc[4][4];
-  ring_product<PE_T, PE_T, 2, 2, 2, false>(A + z * sA, lda, W + z * sW, M, N, K, m0, n0, wv, lane,
-                                           acc, ss);
+  ring_product<PE_T, PE_T, 2, 2, 2, false, EPI == EPI_PE_X>(A + z * sA, lda, W + z * sW, M, N, K,
+                                                            m0, n0, wv, lane, acc, ss, N);
   // chunk q = tid + 256 u of the tile: row q / CPR, columns 8 (q % CPR)
   uint4 xv[EPI == EPI_PE_A ? 1 : NCH];
   if constexpr (EPI != EPI_PE_A) {
@@ -447,9 +489,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       o = make_uint4(w[0], w[1], w[2], w[3]);
       *sy = o;   // kept for a transposed copy
     }
-    *(uint4*)(out + (size_t)(m0 + ml) * ea.ldo + n0 + c8) = o;
+    if (EPI != EPI_PE_X || ea.out) *(uint4*)(out + (size_t)(m0 + ml) * ea.ldo + n0 + c8) = o;
   }
-  // transposed: PE_X's copy x'^T, or the mirror of a tile above the diagonal
+  // transposed: x'^T where PE_X is asked for it, or the mirror of a tile above
+  // the diagonal
   bf16_t* dst = EPI == EPI_PE_X ? (ea.outT ? ea.outT + z * sOut : nullptr)
                                 : (ea.sym && tn != tm ? out : nullptr);
   if (!dst) return;
@@ -474,24 +517,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
 }
 
-// Whole tiles, 16-byte rows, a square output where it is symmetric.
-bool pe_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                  const EpiArgs& ea, long long sA, long long sW, long long sOut, long long sX,
-                  int batch) {
-  if (M % PE_T || N % PE_T || K % RG_BK || K < RG_BK || M < PE_T || N < PE_T) return false;
-  if ((long long)(M / PE_T) * (N / PE_T) * batch > (1 << 30)) return false;
-  if ((lda | ea.ldo) % 8 || ((sA | sW | sOut) & 7) ||
-      (((uintptr_t)A | (uintptr_t)W | (uintptr_t)ea.out) & 15))
-    return false;
-  if (epi != EPI_PE_A && (ea.ldr % 8 || (sX & 7) || ((uintptr_t)ea.x & 15))) return false;
-  if (epi == EPI_PE_X && ea.outT && (ea.ldoT % 8 || ((uintptr_t)ea.outT & 15))) return false;
-  return epi == EPI_PE_X ? !ea.sym : (!ea.sym || M == N);
-}
+// Whole tiles; the strides and bases of the caller (polar_express) are whole
+// matrices of such tiles, 16-byte aligned.
+bool pe_ring_fits(int S, int L) { return S >= PE_T && S % PE_T == 0 && L % PE_T == 0; }
 
 hipError_t pe_ring(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W, long long sW,
                    int M, int N, int K, const EpiArgs& ea, long long sOut, long long sX, int batch,
                    hipStream_t st) {
   const int nbm = M / PE_T, nbn = N / PE_T;
+  if (M % PE_T || N % PE_T || K % RG_BK || K < RG_BK || (ea.sym && M != N) ||
+      (long long)nbm * nbn * batch > (1 << 30))
+    return hipErrorInvalidValue;
   const dim3 grid((ea.sym ? nbm * (nbm + 1) / 2 : nbm * nbn) * batch);
   constexpr size_t lds = rg_lds_bytes<PE_T, PE_T, 2>();   // 64 KB
 #define PE_CASE(E)                                                                              \

@@ -146,14 +146,14 @@ hipError_t gemm_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int
 // Compute units of the current device (256 where the query fails).
 int device_cus();
 // `batch` independent products (sA, sW, sOut, sX: strides of A, W, ea.out /
-// ea.outT, ea.x); epilogues PE_A, PE_B, PE_X.  pe_ring (gemm_ring.hip) where
-// whole 128 x 128 tiles fit, else k_gemm_bat.
-bool pe_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                  const EpiArgs& ea, long long sA, long long sW, long long sOut, long long sX,
-                  int batch);
+// ea.outT, ea.x) of whole 128 x 128 tiles (gemm_ring.hip): epilogues PE_A,
+// PE_B with W (N, K); PE_X with W (K, N), ea.out or ea.outT null where not
+// wanted.  pe_ring_fits: whether the iteration on S x L matrices can use it.
+bool pe_ring_fits(int S, int L);
 hipError_t pe_ring(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W, long long sW,
                    int M, int N, int K, const EpiArgs& ea, long long sOut, long long sX, int batch,
                    hipStream_t st);
+// The same for any shape (W (N, K) for PE_X too): k_gemm_bat.
 hipError_t gemm_batched(int epi, const bf16_t* A, int lda, long long sA, const bf16_t* W,
                         long long sW, int M, int N, int K, const EpiArgs& ea, long long sOut,
                         long long sX, int batch, hipStream_t st);
@@ -171,6 +171,11 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
 size_t normuon_ws_bytes(int batch, int M, int N);
 hipError_t normuon(const bf16_t* v, float* second_mom, int batch, int M, int N, float beta2,
                    float* out, void* ws, size_t ws_bytes, hipStream_t st);
+// normuon and muon_apply on its result in one pass; N % 8 == 0, 16-byte
+// aligned v, p, p_out (p_out may be p).
+hipError_t normuon_update(const bf16_t* v, float* second_mom, int batch, int M, int N, float beta2,
+                          const float* p, float lr, float wd, float* p_out, void* ws,
+                          size_t ws_bytes, hipStream_t st);
 // NorMuon with its scratch in a fixed device array of NM_SCRATCH_BYTES (no
 // allocation; calls that overlap on one GPU race); normuon_ws_bytes(batch, M,
 // N) must not exceed it.

@@ -1258,9 +1258,6 @@ hipError_t gemm_batched(int epi, const bf16_t* A, int lda, long long sA, const b
                         long long sX, int batch, hipStream_t st) {
   if (K % GM_BK != 0 || M <= 0 || N <= 0 || batch <= 0 || batch > 65535)
     return hipErrorInvalidValue;
-  // batches of whole 128 x 128 tiles: the ring
-  if (pe_ring_fits(epi, A, lda, W, M, N, K, ea, sA, sW, sOut, sX, batch))
-    return pe_ring(epi, A, lda, sA, W, sW, M, N, K, ea, sOut, sX, batch, st);
   const int bm = M <= 64 ? 64 : GM_BM;
   dim3 grid((N + GM_BN - 1) / GM_BN, (M + bm - 1) / bm, batch);
 #define ANN_GB(E)                                                                              \

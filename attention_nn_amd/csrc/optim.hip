@@ -6,11 +6,12 @@
 //    weight decay) as the reference kernels.
 //  * Polar Express (muon.py:28-44) on a batch of (M, N) matrices: x = bf16(g /
 //    (||g||_F * 1.02 + 1e-6)), then five iterations of bf16 products on the
-//    MFMA GEMM (batched over blockIdx.z).  Every product is an "NT" GEMM of
-//    k_gemm: x x^T directly; A A because A is symmetric; B x through one
-//    transpose of x per iteration (x B for tall matrices, B symmetric).  The
-//    combinations b A + c A^2 and a x + B x run in the GEMM epilogues with the
-//    eager rounding of each op.
+//    matrix cores.  Shapes of whole 128 x 128 tiles run on the ring kernel
+//    (gemm_ring.hip), a tall matrix transposed; the others on k_gemm_bat, where
+//    every product is an "NT" GEMM: x x^T directly, A A because A is symmetric,
+//    B x through one transpose of x per iteration (x B for tall matrices, B
+//    symmetric).  The combinations b A + c A^2 and a x + B x run in the
+//    epilogues with the eager rounding of each op.
 //  * NorMuon (muon.py:47-63): mean of squares along the reduced axis, one
 //    work-group per matrix for the norms and the second-moment update, then
 //    the broadcast scale.
@@ -138,6 +139,31 @@ __global__ void k_pe_scale(const float* __restrict__ g, size_t mn, const float* 
   }
 }
 
+// X (N, M) = bf16(g / den)^T of g (M, N), 64 x 64 tiles through LDS (M, N
+// multiples of 64): a tall matrix enters the iteration transposed.
+__global__ __launch_bounds__(256) void k_pe_scale_t(const float* __restrict__ g, int M, int N,
+                                                    const float* __restrict__ den,
+                                                    bf16_t* __restrict__ x) {
+  __shared__ bf16_t t[64][64 + 2];
+  const int z = blockIdx.z, r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  const float dz = den[z];
+  const float* s = g + (size_t)z * M * N;
+  bf16_t* d = x + (size_t)z * M * N;
+  const int c4 = (threadIdx.x & 15) * 4;
+  for (int i = threadIdx.x >> 4; i < 64; i += 16) {
+    const float4 v = *(const float4*)(s + (size_t)(r0 + i) * N + c0 + c4);
+    t[c4][i] = f2bf(v.x / dz);
+    t[c4 + 1][i] = f2bf(v.y / dz);
+    t[c4 + 2][i] = f2bf(v.z / dz);
+    t[c4 + 3][i] = f2bf(v.w / dz);
+  }
+  __syncthreads();
+  const int p2 = (threadIdx.x & 31) * 2;
+  for (int i = threadIdx.x >> 5; i < 64; i += 8)
+    *(uint32_t*)(d + (size_t)(c0 + i) * M + r0 + p2) =
+        (uint32_t)t[i][p2] | ((uint32_t)t[i][p2 + 1] << 16);
+}
+
 // dst (C, R) = src (R, C)^T per matrix, 64 x 64 tiles through LDS.
 constexpr int TR_T = 64;
 __global__ __launch_bounds__(256) void k_transpose_bf16(const bf16_t* __restrict__ src,
@@ -206,10 +232,57 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
   bf16_t* bm = (bf16_t*)w;  w += up256(batch * S * S * 2); // B
   float* part = (float*)w;  w += up256(batch * (size_t)nch * 4);
   float* den = (float*)w;
-  // x0 goes to xb so that the fifth (odd) iteration lands in out
   hipLaunchKernelGGL(k_pe_sumsq, dim3(nch, batch), dim3(PE_THREADS), 0, st, g, mn, nch, part);
   hipLaunchKernelGGL(k_pe_norm, dim3(batch), dim3(64), 0, st, part, nch, den);
   const unsigned sg = grid_for(mn / 4, 256);
+  const int Si = (int)S, Li = (int)(mn / S);
+  if (pe_ring_fits(Si, Li) && (((uintptr_t)g | (uintptr_t)out | (uintptr_t)ws) & 15) == 0) {
+    // The iteration on X (S, L), x of a wide matrix or x^T of a tall one
+    // (f(x)^T = f(x^T)): A = X X^T, B = b A + c A A (symmetric: half the tiles),
+    // X' = a X + B X with X itself as the (K, N) operand, so neither x^T nor a
+    // transpose is ever written but a tall result's last step.
+    if (M > N) {
+      hipLaunchKernelGGL(k_pe_scale_t, dim3(N / 64, M / 64, batch), dim3(256), 0, st, g, M, N, den,
+                         xb);
+    } else {
+      hipLaunchKernelGGL(k_pe_scale, dim3(sg < 1024 ? sg : 1024, batch), dim3(256), 0, st, g, mn,
+                         den, xb);
+    }
+    const long long ss = (long long)S * S, sx = (long long)mn;
+    bf16_t* cur = xb;
+    bf16_t* nxt = M > N ? xt : out;   // the fifth (odd) product of a wide matrix lands in out
+    for (int it = 0; it < 5; ++it) {
+      EpiArgs ea{};
+      ea.out = am;
+      ea.ldo = Si;
+      ea.sym = 1;
+      hipError_t e = pe_ring(EPI_PE_A, cur, Li, sx, cur, sx, Si, Si, Li, ea, ss, 0, batch, st);
+      if (e != hipSuccess) return e;
+      ea.out = bm;
+      ea.x = am;
+      ea.ldr = Si;
+      ea.s0 = bf16_round_host(PE_COEF[it][1]);
+      ea.s1 = bf16_round_host(PE_COEF[it][2]);
+      e = pe_ring(EPI_PE_B, am, Si, ss, am, ss, Si, Si, Si, ea, ss, ss, batch, st);
+      if (e != hipSuccess) return e;
+      const bool last_tall = it == 4 && M > N;
+      ea.sym = 0;
+      ea.out = last_tall ? nullptr : nxt;
+      ea.ldo = Li;
+      ea.outT = last_tall ? out : nullptr;
+      ea.ldoT = Si;
+      ea.x = cur;
+      ea.ldr = Li;
+      ea.s0 = bf16_round_host(PE_COEF[it][0]);
+      e = pe_ring(EPI_PE_X, bm, Si, ss, cur, sx, Si, Li, Si, ea, sx, sx, batch, st);
+      if (e != hipSuccess) return e;
+      bf16_t* t = cur;
+      cur = nxt;
+      nxt = t;
+    }
+    return hipGetLastError();
+  }
+  // other shapes: x0 goes to xb so that the fifth (odd) iteration lands in out
   hipLaunchKernelGGL(k_pe_scale, dim3(sg < 1024 ? sg : 1024, batch), dim3(256), 0, st, g, mn, den,
                      xb);
   bf16_t* cur = xb;
@@ -226,11 +299,9 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
     EpiArgs ea{};
     hipError_t e;
     if (!tall) {
-      // A = x x^T (M x M, K = N); A and B below are symmetric: only the tiles
-      // on and above the diagonal are computed (their mirrors stored transposed)
+      // A = x x^T (M x M, K = N)
       ea.out = am;
       ea.ldo = M;
-      ea.sym = 1;
       e = gemm_batched(EPI_PE_A, cur, N, (long long)mn, cur, (long long)mn, M, M, N, ea,
                        (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
@@ -244,7 +315,6 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
                        (long long)S * S, (long long)S * S, batch, st);
       if (e != hipSuccess) return e;
       // x' = a x + B x: B (M x M) against x^T (N x M)
-      ea.sym = 0;
       ea.out = nxt;
       ea.ldo = N;
       ea.x = cur;
@@ -256,10 +326,9 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
                        (long long)mn, (long long)mn, batch, st);
       if (e != hipSuccess) return e;
     } else {
-      // A = x^T x (N x N, K = M) from x^T (N x M); A and B symmetric as above
+      // A = x^T x (N x N, K = M) from x^T (N x M)
       ea.out = am;
       ea.ldo = N;
-      ea.sym = 1;
       e = gemm_batched(EPI_PE_A, xt, M, (long long)mn, xt, (long long)mn, N, N, M, ea,
                        (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
@@ -271,7 +340,6 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       e = gemm_batched(EPI_PE_B, am, N, (long long)S * S, am, (long long)S * S, N, N, N, ea,
                        (long long)S * S, (long long)S * S, batch, st);
       if (e != hipSuccess) return e;
-      ea.sym = 0;
       // x' = a x + x B (B symmetric: its rows are the columns of B)
       ea.out = nxt;
       ea.ldo = N;
@@ -394,16 +462,47 @@ __global__ void k_nm_apply(const bf16_t* __restrict__ v, int M, int N, int rows,
   }
 }
 
+// The scale and muon_apply in one pass: u = v * scale[line] stays in a register
+// (the same products as the two kernels: 4 + 4 bytes per value less traffic;
+// 52 us a 155M bank against 59 + 58).
+// Eight values per thread: N % 8 == 0, 16-byte aligned p and po, v.
+__global__ __launch_bounds__(256) void k_nm_update(const bf16_t* __restrict__ v, int N, int rows,
+                                                   size_t mn, const float* __restrict__ scale,
+                                                   int R, const float* __restrict__ p, float lr,
+                                                   float wd, float* __restrict__ po) {
+  const int z = blockIdx.y;
+  const float* sz = scale + (size_t)z * R;
+  const unsigned n8 = (unsigned)(mn / 8), nr8 = (unsigned)N / 8, stride = gridDim.x * blockDim.x;
+  const uint4* v4 = (const uint4*)(v + z * mn);
+  const float4* p4 = (const float4*)(p + z * mn);
+  float4* o4 = (float4*)(po + z * mn);
+  for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += stride) {
+    const unsigned row = i / nr8, c8 = (i - row * nr8) * 8;
+    const uint4 vw = v4[i];
+    const float4 pa = p4[2 * (size_t)i], pb = p4[2 * (size_t)i + 1];
+    float f[8], q[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+    unpack8(vw, f);
+    const float sr = rows ? sz[row] : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float u = f[e] * (rows ? sr : sz[c8 + e]);
+      if (u * q[e] >= 0.0f) q[e] -= q[e] * wd * lr;
+      q[e] -= u * lr;
+    }
+    o4[2 * (size_t)i] = make_float4(q[0], q[1], q[2], q[3]);
+    o4[2 * (size_t)i + 1] = make_float4(q[4], q[5], q[6], q[7]);
+  }
+}
+
 size_t normuon_ws_bytes(int batch, int M, int N) {
   const size_t R = M >= N ? M : N;
   return batch > 0 ? 2 * up256((size_t)batch * R * 4) : 0;
 }
 
-hipError_t normuon(const bf16_t* v, float* second_mom, int batch, int M, int N, float beta2,
-                   float* out, void* ws, size_t ws_bytes, hipStream_t st) {
-  if (batch <= 0 || M <= 0 || N <= 0 || !v || !second_mom || !out || !ws ||
-      ws_bytes < normuon_ws_bytes(batch, M, N))
-    return hipErrorInvalidValue;
+// Line means, the second-moment update and the per-line scales (in ws); the
+// scales' address in *scale.
+static hipError_t normuon_scales(const bf16_t* v, float* second_mom, int batch, int M, int N,
+                                 float beta2, void* ws, float** scale, hipStream_t st) {
   const bool rows = M >= N;
   const int R = rows ? M : N, red = rows ? N : M;
   float* vm = (float*)ws;
@@ -415,8 +514,38 @@ hipError_t normuon(const bf16_t* v, float* second_mom, int batch, int M, int N, 
                        vm);
   hipLaunchKernelGGL(k_nm_scale, dim3(batch), dim3(NM_THREADS), 0, st, vm, R, red, beta2,
                      second_mom, sc);
+  *scale = sc;
+  return hipGetLastError();
+}
+
+hipError_t normuon(const bf16_t* v, float* second_mom, int batch, int M, int N, float beta2,
+                   float* out, void* ws, size_t ws_bytes, hipStream_t st) {
+  if (batch <= 0 || M <= 0 || N <= 0 || !v || !second_mom || !out || !ws ||
+      ws_bytes < normuon_ws_bytes(batch, M, N))
+    return hipErrorInvalidValue;
+  float* sc = nullptr;
+  const hipError_t e = normuon_scales(v, second_mom, batch, M, N, beta2, ws, &sc, st);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_nm_apply, dim3(grid_for((size_t)batch * M * N, 256)), dim3(256), 0, st, v,
-                     M, N, (int)rows, sc, out, batch);
+                     M, N, (int)(M >= N), sc, out, batch);
+  return hipGetLastError();
+}
+
+hipError_t normuon_update(const bf16_t* v, float* second_mom, int batch, int M, int N, float beta2,
+                          const float* p, float lr, float wd, float* p_out, void* ws,
+                          size_t ws_bytes, hipStream_t st) {
+  const size_t mn = (size_t)M * N;
+  if (batch <= 0 || batch > 65535 || M <= 0 || N <= 0 || N % 8 || mn >= ((size_t)1 << 33) || !v ||
+      !second_mom || !p || !p_out || !ws || ws_bytes < normuon_ws_bytes(batch, M, N) ||
+      (((uintptr_t)v | (uintptr_t)p | (uintptr_t)p_out) & 15))
+    return hipErrorInvalidValue;
+  float* sc = nullptr;
+  const hipError_t e = normuon_scales(v, second_mom, batch, M, N, beta2, ws, &sc, st);
+  if (e != hipSuccess) return e;
+  unsigned g = grid_for(mn / 8, 256);
+  if (g > 8192) g = 8192;
+  hipLaunchKernelGGL(k_nm_update, dim3(g, batch), dim3(256), 0, st, v, N, (int)(M >= N), mn, sc,
+                     M >= N ? M : N, p, lr, wd, p_out);
   return hipGetLastError();
 }
 

@@ -221,6 +221,14 @@ size_t ann_op_normuon_ws_bytes(int32_t batch, int32_t M, int32_t N);
 int ann_op_normuon(const void* v, float* second_mom, int32_t batch, int32_t M, int32_t N,
                    float beta2, float* out, void* ws, size_t ws_bytes, void* stream);
 
+/* normuon_rescale and muon_apply in one pass (muon.py:121-127): the rescaled
+ * update u is not stored, p' = p - p*wd*lr (where u*p >= 0) - u*lr.  N a
+ * multiple of 8; v, p and p_out 16-byte aligned; p_out may be p; ws:
+ * ann_op_normuon_ws_bytes(batch, M, N). */
+int ann_op_normuon_update(const void* v, float* second_mom, int32_t batch, int32_t M, int32_t N,
+                          float beta2, const float* p, float lr, float wd, float* p_out, void* ws,
+                          size_t ws_bytes, void* stream);
+
 /* NorMuon without an allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight training or serving loops, harnesses that forbid hipMalloc).  Same

@@ -1,0 +1,32 @@
+"""NorMuon and the parameter update in one pass against the two operators it
+stands for, bit for bit: wide, tall, square and single-line shapes, a last
+dimension that is no multiple of 8 and an unaligned parameter (both take the
+two operators)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 192), (3, 192, 64), (1, 128, 128), (2, 8, 8), (1, 1, 24),
+                                   (5, 24, 8), (2, 12, 10), (2, 6, 28)])
+def test_update_equals_rescale_then_apply(shape):
+    from attention_nn_amd import optim as G
+    g = torch.Generator().manual_seed(sum(shape))
+    v = torch.randn(shape, generator=g).bfloat16().cuda()
+    p = torch.randn(shape, generator=g).cuda()
+    M, N = shape[-2:]
+    line = (shape[0], M, 1) if M >= N else (shape[0], 1, N)
+    sm = (torch.rand(line, generator=g) * 0.1).cuda()
+    buf = torch.empty(p.numel() + 1, device="cuda")
+    odd = buf[1:].view(shape)
+    odd.copy_(p)
+    u, rsm = G.normuon_rescale(v, sm, 0.9)
+    ref = G.muon_apply(p, u, 0.02, 1.2)
+    for q in (p, odd):
+        got, gsm = G._normuon_update(v, sm, 0.9, q, 0.02, 1.2)
+        assert torch.equal(got, ref) and torch.equal(gsm, rsm)
+    with pytest.raises(ValueError):
+        G._normuon_update(v, sm, 0.9, p[..., :N // 2].contiguous(), 0.02, 1.2) if N % 8 == 0 \
+            else G.normuon_rescale(v, sm.reshape(-1)[1:], 0.9)
