@@ -1,7 +1,7 @@
 """NorMuon and the parameter update in one pass against the two operators it
 stands for, bit for bit: wide, tall, square and single-line shapes, a last
 dimension that is no multiple of 8 and an unaligned parameter (both take the
-two operators)."""
+two operators), a parameter of other leading dimensions."""
 
 import pytest
 import torch
@@ -27,6 +27,8 @@ def test_update_equals_rescale_then_apply(shape):
     for q in (p, odd):
         got, gsm = G._normuon_update(v, sm, 0.9, q, 0.02, 1.2)
         assert torch.equal(got, ref) and torch.equal(gsm, rsm)
+    flat, _ = G._normuon_update(v, sm, 0.9, p.reshape(-1, N), 0.02, 1.2)
+    assert flat.shape == (p.numel() // N, N) and torch.equal(flat.view(shape), ref)
     with pytest.raises(ValueError):
         G._normuon_update(v, sm, 0.9, p[..., :N // 2].contiguous(), 0.02, 1.2) if N % 8 == 0 \
             else G.normuon_rescale(v, sm.reshape(-1)[1:], 0.9)
