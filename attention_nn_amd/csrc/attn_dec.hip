@@ -359,7 +359,7 @@ void k_attn_dec(
 }
 
 // The decode step's RMS + qkv projection and its attention in one launch
-// (batch 16..64, d <= 768, direct launches only): work-groups [0, ngemm) run
+// (batch 4..64, d <= 768, direct launches only): work-groups [0, ngemm) run
 // the skinny GEMM's 16T x 16T tiles (gemm_sk_body, the same arithmetic as
 // k_gemm_sk) and publish bf16 pairs of q, k, v as tagged words xt[m][n / 2]
 // (tag = this launch's, from a host counter that only grows); the attention

@@ -410,7 +410,7 @@ int run_body(ann_ctx* c, const int32_t* tokens, int B, int T, hipStream_t st) {
         fuse_qkv = true;
       }
     }
-    // decode of 16..64 rows launched directly: the qkv projection and the
+    // decode of 4..64 rows launched directly: the qkv projection and the
     // attention as one launch (qkv_attn_decode); never inside a graph
     // capture (its tag comes from a host counter) or a per-kernel profile
     bool fuse_qa = T == 1 && c->qa_env && c->prof_kind < 0 && qkv_attn_fits(B, d, Dh);
@@ -1071,7 +1071,12 @@ int ann_decode_step(ann_ctx* c, const int32_t* tokens, int32_t B, const ann_samp
   // GRAPH_MAX_B rows; from there launched directly, ~4 us per step faster
   // (batch 64 557.4 -> 553.0 us, 16 x 8192 504.1 -> 500.1, 128 rows equal),
   // the host enqueueing a step well inside its GPU time.
-  const bool graph = c->graph_mode == 1 || (c->graph_mode < 0 && B < GRAPH_MAX_B);
+  // So are fewer rows whose qkv projection and attention can be one launch,
+  // which a graph cannot hold: 155M, 7 rows of 150 tokens and 48 steps 15.80 ->
+  // 14.99 ms (a step 310 -> 293 us).
+  const bool graph = c->graph_mode == 1 ||
+                     (c->graph_mode < 0 && B < GRAPH_MAX_B &&
+                      !(c->qa_env && qkv_attn_fits(B, c->c.d, c->Dh)));
   if (graph && c->prof_kind < 0 && !persist_ok(c, B))
     rc = decode_graph(c, tokens, B, greedy, out_tok, logits, st);
   else
