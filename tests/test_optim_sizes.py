@@ -1,5 +1,6 @@
-"""Optimizer operators whose tensors do not belong together: refused on the
-host, before anything is launched (the library raises on any use here)."""
+"""The optimizer's host checks: tensors that do not belong together are refused
+before anything is launched (the library raises on any use here), and a matrix
+beyond the one-pass update's range takes the two operators."""
 
 import pytest
 import torch
@@ -45,3 +46,12 @@ def test_update_of_another_size_than_the_parameter(N, param):
             G._normuon_update(v, sm, 0.9, param(shape), 0.02, 1.2)
     with pytest.raises(ValueError, match="belong together"):
         G._normuon_update(v, sm[:1], 0.9, param((2, 8, N)), 0.02, 1.2)
+
+
+def test_matrix_beyond_the_one_pass_update_takes_the_two_operators(monkeypatch):
+    v = torch.empty((1, 1 << 17, 1 << 16), dtype=torch.bfloat16, device="meta")
+    p, sm = torch.empty(v.shape, device="meta"), torch.empty((1, 1 << 17, 1), device="meta")
+    monkeypatch.setattr(G, "normuon_rescale", lambda v, sm, beta2: ("u", sm))
+    monkeypatch.setattr(G, "muon_apply", lambda p, u, lr, wd: (u, lr, wd))
+    got, gsm = G._normuon_update(v, sm, 0.9, p, 0.02, 1.2)
+    assert got == ("u", 0.02, 1.2) and gsm is sm
