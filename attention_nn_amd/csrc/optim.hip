@@ -465,11 +465,12 @@ __global__ void k_nm_apply(const bf16_t* __restrict__ v, int M, int N, int rows,
 // The scale and muon_apply in one pass: u = v * scale[line] stays in a register
 // (the same products as the two kernels: 4 + 4 bytes per value less traffic;
 // 52 us a 155M bank against 59 + 58).
-// Eight values per thread: N % 8 == 0, 16-byte aligned p and po, v.
+// Eight values per thread: N % 8 == 0, 16-byte aligned p and po, v.  po may be
+// p: a thread reads its words before it writes them, and no other's.
 __global__ __launch_bounds__(256) void k_nm_update(const bf16_t* __restrict__ v, int N, int rows,
                                                    size_t mn, const float* __restrict__ scale,
-                                                   int R, const float* __restrict__ p, float lr,
-                                                   float wd, float* __restrict__ po) {
+                                                   int R, const float* p, float lr, float wd,
+                                                   float* po) {
   const int z = blockIdx.y;
   const float* sz = scale + (size_t)z * R;
   const unsigned n8 = (unsigned)(mn / 8), nr8 = (unsigned)N / 8, stride = gridDim.x * blockDim.x;

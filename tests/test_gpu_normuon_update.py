@@ -1,7 +1,8 @@
 """NorMuon and the parameter update in one pass against the two operators it
 stands for, bit for bit: wide, tall, square and single-line shapes, a last
 dimension that is no multiple of 8 and an unaligned parameter (both take the
-two operators), a parameter of other leading dimensions."""
+two operators), a parameter of other leading dimensions, and the C entry
+writing over the parameter it reads."""
 
 import pytest
 import torch
@@ -32,3 +33,21 @@ def test_update_equals_rescale_then_apply(shape):
     with pytest.raises(ValueError):
         G._normuon_update(v, sm, 0.9, p[..., :N // 2].contiguous(), 0.02, 1.2) if N % 8 == 0 \
             else G.normuon_rescale(v, sm.reshape(-1)[1:], 0.9)
+
+
+@pytest.mark.parametrize("shape", [(2, 64, 192), (3, 192, 64), (1, 1, 24), (1, 768, 3072)])
+def test_update_in_place(shape):
+    from attention_nn_amd import _lib, optim as G
+    from attention_nn_amd._stream import current_stream
+    batch, M, N = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    v = torch.randn(shape, generator=g).bfloat16().cuda()
+    p = torch.randn(shape, generator=g).cuda()
+    sm = (torch.rand((batch, max(M, N)), generator=g) * 0.1).cuda()
+    ref, _ = G._normuon_update(v, sm, 0.9, p, 0.02, 1.2)
+    nws = _lib.lib().ann_op_normuon_ws_bytes(batch, M, N)
+    ws = torch.empty(nws, dtype=torch.uint8, device="cuda")
+    _lib.check(_lib.lib().ann_op_normuon_update(G._ptr(v), G._ptr(sm), batch, M, N, 0.9, G._ptr(p),
+                                                0.02, 1.2, G._ptr(p), G._ptr(ws), nws,
+                                                current_stream()))
+    assert torch.equal(p, ref)
