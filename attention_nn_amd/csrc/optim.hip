@@ -10,7 +10,8 @@
 //    (gemm_ring.hip), a tall matrix transposed; the others on k_gemm_bat, where
 //    every product is an "NT" GEMM: x x^T directly, A A because A is symmetric,
 //    B x through one transpose of x per iteration (x B for tall matrices, B
-//    symmetric).  The combinations b A + c A^2 and a x + B x run in the
+//    symmetric); their A and B still run on the ring kernel where the shorter
+//    side is whole tiles (22 x 768 x 2880: 1839 -> 1305 us).  The combinations b A + c A^2 and a x + B x run in the
 //    epilogues with the eager rounding of each op.
 //  * NorMuon (muon.py:47-63): mean of squares along the reduced axis, one
 //    work-group per matrix for the norms and the second-moment update, then
@@ -164,6 +165,11 @@ __global__ __launch_bounds__(256) void k_pe_scale_t(const float* __restrict__ g,
         (uint32_t)t[i][p2] | ((uint32_t)t[i][p2 + 1] << 16);
 }
 
+__global__ void k_copy_bf16(const bf16_t* __restrict__ src, bf16_t* __restrict__ dst, size_t n) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
+}
+
 // dst (C, R) = src (R, C)^T per matrix, 64 x 64 tiles through LDS.
 constexpr int TR_T = 64;
 __global__ __launch_bounds__(256) void k_transpose_bf16(const bf16_t* __restrict__ src,
@@ -236,7 +242,9 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
   hipLaunchKernelGGL(k_pe_norm, dim3(batch), dim3(64), 0, st, part, nch, den);
   const unsigned sg = grid_for(mn / 4, 256);
   const int Si = (int)S, Li = (int)(mn / S);
-  if (pe_ring_fits(Si, Li) && (((uintptr_t)g | (uintptr_t)out | (uintptr_t)ws) & 15) == 0) {
+  auto aligned = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
+  // (g's 16-byte loads need its own four bytes only)
+  if (pe_ring_fits(Si, Li) && aligned(ws)) {
     // The iteration on X (S, L), x of a wide matrix or x^T of a tall one
     // (f(x)^T = f(x^T)): A = X X^T, B = b A + c A A (symmetric: half the tiles),
     // X' = a X + B X with X itself as the (K, N) operand, so neither x^T nor a
@@ -248,9 +256,13 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       hipLaunchKernelGGL(k_pe_scale, dim3(sg < 1024 ? sg : 1024, batch), dim3(256), 0, st, g, mn,
                          den, xb);
     }
+    // a result that is not 16-byte aligned is formed in the workspace (xt2, which
+    // this form does not use otherwise) and copied: 22 x 768 x 3072 1025 us, on
+    // k_gemm_bat 2925
+    bf16_t* res = aligned(out) ? out : xt2;
     const long long ss = (long long)S * S, sx = (long long)mn;
     bf16_t* cur = xb;
-    bf16_t* nxt = M > N ? xt : out;   // the fifth (odd) product of a wide matrix lands in out
+    bf16_t* nxt = M > N ? xt : res;   // the fifth (odd) product of a wide matrix lands in res
     for (int it = 0; it < 5; ++it) {
       EpiArgs ea{};
       ea.out = am;
@@ -269,7 +281,7 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       ea.sym = 0;
       ea.out = last_tall ? nullptr : nxt;
       ea.ldo = Li;
-      ea.outT = last_tall ? out : nullptr;
+      ea.outT = last_tall ? res : nullptr;
       ea.ldoT = Si;
       ea.x = cur;
       ea.ldr = Li;
@@ -280,9 +292,18 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       cur = nxt;
       nxt = t;
     }
+    if (res != out)
+      hipLaunchKernelGGL(k_copy_bf16, dim3(grid_for(batch * mn, 256)), dim3(256), 0, st, res, out,
+                         batch * mn);
     return hipGetLastError();
   }
-  // other shapes: x0 goes to xb so that the fifth (odd) iteration lands in out
+  // Other shapes: x0 goes to xb so that the fifth (odd) iteration lands in out.
+  // Where the shorter side is whole 128-tiles and the operands are aligned, A and
+  // B still come from the ring kernel, half their tiles each (their K may be any
+  // multiple of 64).
+  auto half_tiles = [&](const bf16_t* x) {
+    return pe_ring_fits(Si, Si) && aligned(ws) && aligned(x);
+  };
   hipLaunchKernelGGL(k_pe_scale, dim3(sg < 1024 ? sg : 1024, batch), dim3(256), 0, st, g, mn, den,
                      xb);
   bf16_t* cur = xb;
@@ -302,8 +323,9 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       // A = x x^T (M x M, K = N)
       ea.out = am;
       ea.ldo = M;
-      e = gemm_batched(EPI_PE_A, cur, N, (long long)mn, cur, (long long)mn, M, M, N, ea,
-                       (long long)S * S, 0, batch, st);
+      ea.sym = half_tiles(cur);
+      e = (ea.sym ? pe_ring : gemm_batched)(EPI_PE_A, cur, N, (long long)mn, cur, (long long)mn, M,
+                                            M, N, ea, (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
       // B = b A + c (A A)
       ea.out = bm;
@@ -311,10 +333,13 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       ea.ldr = M;
       ea.s0 = b;
       ea.s1 = c;
-      e = gemm_batched(EPI_PE_B, am, M, (long long)S * S, am, (long long)S * S, M, M, M, ea,
-                       (long long)S * S, (long long)S * S, batch, st);
+      ea.sym = half_tiles(am);
+      e = (ea.sym ? pe_ring : gemm_batched)(EPI_PE_B, am, M, (long long)S * S, am,
+                                            (long long)S * S, M, M, M, ea, (long long)S * S,
+                                            (long long)S * S, batch, st);
       if (e != hipSuccess) return e;
       // x' = a x + B x: B (M x M) against x^T (N x M)
+      ea.sym = 0;
       ea.out = nxt;
       ea.ldo = N;
       ea.x = cur;
@@ -329,18 +354,22 @@ hipError_t polar_express(const float* g, int batch, int M, int N, bf16_t* out, v
       // A = x^T x (N x N, K = M) from x^T (N x M)
       ea.out = am;
       ea.ldo = N;
-      e = gemm_batched(EPI_PE_A, xt, M, (long long)mn, xt, (long long)mn, N, N, M, ea,
-                       (long long)S * S, 0, batch, st);
+      ea.sym = half_tiles(xt);
+      e = (ea.sym ? pe_ring : gemm_batched)(EPI_PE_A, xt, M, (long long)mn, xt, (long long)mn, N,
+                                            N, M, ea, (long long)S * S, 0, batch, st);
       if (e != hipSuccess) return e;
       ea.out = bm;
       ea.x = am;
       ea.ldr = N;
       ea.s0 = b;
       ea.s1 = c;
-      e = gemm_batched(EPI_PE_B, am, N, (long long)S * S, am, (long long)S * S, N, N, N, ea,
-                       (long long)S * S, (long long)S * S, batch, st);
+      ea.sym = half_tiles(am);
+      e = (ea.sym ? pe_ring : gemm_batched)(EPI_PE_B, am, N, (long long)S * S, am,
+                                            (long long)S * S, N, N, N, ea, (long long)S * S,
+                                            (long long)S * S, batch, st);
       if (e != hipSuccess) return e;
       // x' = a x + x B (B symmetric: its rows are the columns of B)
+      ea.sym = 0;
       ea.out = nxt;
       ea.ldo = N;
       ea.x = cur;

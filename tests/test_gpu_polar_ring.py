@@ -1,9 +1,12 @@
 """Polar Express on the ring products (gemm_ring.hip): one tile, symmetric
 outputs of two and three tiles (mirrored tiles), wide, tall and batched banks,
-and shapes of 64 but not 128 (the general tiles) beside them."""
+and shapes of 64 but not 128 (the general tiles) beside them; half the tiles of
+A and B wherever the shorter side is whole tiles, aligned buffers or not."""
 
 import pytest
 import torch
+
+from torch.profiler import ProfilerActivity, profile
 
 import oracle.ref_optim as O
 
@@ -26,3 +29,48 @@ def test_polar_ring_matches_oracle(shape):
     assert rel < 4e-2, rel
     for z in range(shape[0]):
         assert torch.equal(G.polar_express(g[z:z + 1].cuda())[0], got[z])
+
+
+def _launches(fn, name):
+    """How many kernels of that name one call of fn launches."""
+    fn()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return sum(name in e.name for e in prof.events())
+
+
+def _polar_into(g, out):
+    from attention_nn_amd import _lib
+    from attention_nn_amd import optim as G
+    from attention_nn_amd._stream import current_stream
+    batch, M, N = g.shape
+    nws = _lib.lib().ann_op_polar_express_ws_bytes(batch, M, N)
+    ws = torch.empty(nws, dtype=torch.uint8, device="cuda")
+    _lib.check(_lib.lib().ann_op_polar_express(G._ptr(g), batch, M, N, G._ptr(out), G._ptr(ws), nws,
+                                               current_stream()))
+    return out
+
+
+@pytest.mark.parametrize("shape", [(2, 128, 192), (2, 320, 256), (1, 256, 320), (2, 384, 128),
+                                   (1, 128, 384), (1, 192, 256)])
+@pytest.mark.parametrize("off_g,off_out", [(0, 0), (1, 0), (0, 1)])
+def test_polar_symmetric_products_take_half_their_tiles(shape, off_g, off_out):
+    """The five A and five B products on k_pe_ring where the shorter side is
+    whole tiles; buffers at any element give the bits of aligned ones."""
+    S, n = min(shape[1:]), torch.Size(shape).numel()
+    torch.manual_seed(n)
+    ref_in = torch.randn(shape).cuda()
+    ref = _polar_into(ref_in, torch.empty(shape, dtype=torch.bfloat16, device="cuda"))
+    g = torch.empty(n + 1, device="cuda")[off_g:off_g + n].view(shape).copy_(ref_in)
+    out = torch.zeros(n + 1, dtype=torch.bfloat16, device="cuda")[off_out:off_out + n].view(shape)
+    print(f"case polar half tiles {shape} {off_g} {off_out}", flush=True)
+    assert torch.equal(_polar_into(g, out), ref)
+    # a wide matrix's A of the second and fourth x reads the result buffer itself,
+    # which the general path only takes aligned
+    skipped = 2 if off_out and shape[1] < shape[2] and max(shape[1:]) % 128 else 0
+    half = S % 128 == 0
+    for epi in (10, 7):
+        got = _launches(lambda: _polar_into(g, out), f"k_pe_ring<{epi}>")
+        assert got == (5 - (skipped if epi == 10 else 0) if half else 0)
