@@ -279,7 +279,7 @@ int proj(ann_ctx* c, int kind, int epi, int pre, const bf16_t* W, const bf16_t* 
   if (pre == PRE_RMS && !use_gemv && !use_sk && gemm_ring_fits(epi, X, ldx, W, M, N, K, ea) &&
       gemm_ring_rms(epi, M, N, K)) {
     ProfScope ps(c, kind, st);
-    HIPCHK(gemm_ring(epi, X, ldx, W, M, N, K, ea, st));
+    HIPCHK(gemm_ring(epi, true, X, ldx, W, M, N, K, ea, st));
     return ANN_OK;
   }
   // 65-128 rows with an RMS prologue and a plain-store epilogue (qkv, fc):

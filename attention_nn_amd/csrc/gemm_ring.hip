@@ -145,8 +145,8 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[j][i] = (rg_floatx4){0.f, 0.f, 0.f, 0.f};
 
-  // the k steps of 32 run in order, as in every GEMM here: the same bits
-  // whatever the tile
+  // the k steps of 32 run in order, as in every GEMM here: one product has the
+  // same bits whatever the tile (of rms(A): those of the tiles that form it)
   const int r16 = lane & 15, kg = lane >> 4, sw = (r16 >> 1) & 7;
   const int wm = wv / WC, wn = wv % WC;
   const int oa = (wm * WM + r16) * RG_RB, ow = BM * RG_RB + (wn * WN + r16) * RG_RB;
@@ -239,7 +239,9 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
   // prompts of 777 / 300 tokens 690 -> 647 and 594 -> 547 us.  The large tiles
   // have no issue slots for that (d 1536, 128 x 1024 tokens and 24 steps: 36.55
   // ms with it, 35.80 without).  The lm_head always takes the
-  // rounded rms(x), so that z is the same bits on every route to it.
+  // rounded rms(x), so that z is the same bits on every route to it.  Which of
+  // the two A is comes from the caller (gemm_ring's rms): for a plain A the small
+  // tiles of these epilogues are not picked.
   constexpr bool RMS = ring_takes_rms(EPI, BM, BN);
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && BM * CPR % TH == 0, "whole loads");
   static_assert(EPI != EPI_QKV || (BN == 128 && TH == 256), "whole heads per tile");
@@ -586,19 +588,26 @@ constexpr int RING_N = 5, RING_QKV_N = 7;
 
 }  // namespace
 
+// Whether tile t can run the epilogue on an A taken as it is (plain), or on
+// either A: the qkv and fc epilogues of the small tiles exist with the rms only.
+static bool ring_has(const RingTile& t, int i, int epi, bool plain) {
+  if (epi == EPI_QKV ? t.bn != 128 : i >= RING_N) return false;
+  if (epi == EPI_CE && t.bn < 128) return false;   // partial sums of at most V / 128 tiles
+  return !(plain && ring_takes_rms(epi, t.bm, t.bn));
+}
+
 // The tile that is done first: the CU with the most work-groups takes them in
 // pairs (two are resident).  Measured against every tile at 130 .. 32768 rows
 // of d 512, 768 and 1536: within 5% of the best one at most shapes, 15% at
-// the worst.  One always fits (N is a multiple of 64, of 128 for QKV).
-static int ring_pick(int epi, int M, int N, int K) {
+// the worst.  -1 where no tile divides N (of any A: N is a multiple of 64, of
+// 128 for QKV; plain qkv and fc: of 128 or 192).
+static int ring_pick(int epi, bool plain, int M, int N, int K) {
   static const int cus = device_cus();
   int best = -1;
   long long best_ns = 0;
   for (int i = 0; i < RING_QKV_N; ++i) {
     const RingTile& t = RING_TILES[i];
-    if (epi == EPI_QKV ? t.bn != 128 : i >= RING_N) continue;
-    if (epi == EPI_CE && t.bn < 128) continue;   // partial sums of at most V / 128 tiles
-    if (N % t.bn) continue;
+    if (!ring_has(t, i, epi, plain) || N % t.bn) continue;
     const long long wgs = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn);
     const long long n = (wgs + cus - 1) / cus;
     const long long ns = K / RG_BK * (n / 2 * 2 * t.shared + n % 2 * t.alone) + t.fixed;
@@ -608,6 +617,11 @@ static int ring_pick(int epi, int M, int N, int K) {
     }
   }
   return best;
+}
+
+int gemm_ring_tile(int epi, bool rms, int M, int N, int K) {
+  const int i = ring_pick(epi, !rms, M, N, K);
+  return i < 0 ? 0 : RING_TILES[i].bm << 16 | RING_TILES[i].bn;
 }
 
 // Rows of A and of the epilogue's operands in 16-byte words, whole 64-column
@@ -639,13 +653,14 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
 
 int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                  const EpiArgs& ea) {
-  return gemm_ring_fits(EPI_CE, A, lda, W, M, N, K, ea) ? RING_TILES[ring_pick(EPI_CE, M, N, K)].bn
-                                                        : 128;
+  return gemm_ring_fits(EPI_CE, A, lda, W, M, N, K, ea)
+             ? RING_TILES[ring_pick(EPI_CE, true, M, N, K)].bn
+             : 128;
 }
 
 bool gemm_ring_rms(int epi, int M, int N, int K) {
-  const RingTile& t = RING_TILES[ring_pick(epi, M, N, K)];
-  return ring_takes_rms(epi, t.bm, t.bn);
+  const int i = ring_pick(epi, false, M, N, K);
+  return i >= 0 && ring_takes_rms(epi, RING_TILES[i].bm, RING_TILES[i].bn);
 }
 
 hipError_t gemm_ring_prepare() {
@@ -658,12 +673,13 @@ hipError_t gemm_ring_prepare() {
   return ok ? hipSuccess : hipErrorInvalidValue;
 }
 
-hipError_t gemm_ring(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                     const EpiArgs& ea, hipStream_t st) {
-  if (!gemm_ring_fits(epi, A, lda, W, M, N, K, ea)) return hipErrorInvalidValue;
+hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* W, int M, int N,
+                     int K, const EpiArgs& ea, hipStream_t st) {
+  if (!gemm_ring_fits(epi, A, lda, W, M, N, K, ea) || (rms && !gemm_ring_rms(epi, M, N, K)))
+    return hipErrorInvalidValue;
   const hipError_t e = gemm_ring_prepare();
   if (e != hipSuccess) return e;
-  const int tile = ring_pick(epi, M, N, K);
+  const int tile = ring_pick(epi, !rms, M, N, K);   // none (-1) falls through to the error
 #define RING_TILE(E, T, BM, BN, NS, WR, WC) \
   case T: return launch_ring<E, BM, BN, NS, WR, WC>(A, lda, W, M, N, K, ea, st);
 #define RING(E)                         \

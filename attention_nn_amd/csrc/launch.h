@@ -121,14 +121,16 @@ bool gemm_skinny_fits(int M, int N, int K, bool rms);
 bool gemm_qkv_fits(int M, int N, int K, const EpiArgs& ea);
 // Projections of the prefill, the training forward and whole-context logits:
 // 32 x 64 .. 128 x 192 tiles by shape, K tiles streamed into an LDS ring
-// (gemm_ring.hip).  y = a @ W^T; where gemm_ring_rms says so (EPI_STORE,
-// EPI_RELU2 and EPI_QKV on the small tiles) y = rms(a) @ W^T over rows of K
-// values (ea.eps).
+// (gemm_ring.hip).  y = a @ W^T, or with `rms` y = rms(a) @ W^T over rows of K
+// values (ea.eps), which is only there where gemm_ring_rms says so (EPI_STORE,
+// EPI_RELU2 and EPI_QKV whose fastest tile is a small one).
 bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                     const EpiArgs& ea);
 bool gemm_ring_rms(int epi, int M, int N, int K);
-hipError_t gemm_ring(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                     const EpiArgs& ea, hipStream_t st);
+hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* W, int M, int N,
+                     int K, const EpiArgs& ea, hipStream_t st);
+// The tile it takes: rows << 16 | columns, 0 where there is none.
+int gemm_ring_tile(int epi, bool rms, int M, int N, int K);
 // Columns of gemm_ring's EPI_CE tiles (of gemm()'s, 128, where the ring does
 // not fit): ceil(N / columns) partial sums per row.
 int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
@@ -190,8 +192,8 @@ hipError_t gemm_skinny(int epi, bool rms, const bf16_t* A, int lda, const bf16_t
                        int K, float eps, const EpiArgs& ea, hipStream_t st);
 hipError_t gemm_decode64(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                          const EpiArgs& ea, hipStream_t st);
-// MFMA GEMM: y = A @ W^T with A (M, lda) bf16 (as gemm_ring where that takes
-// the shape).
+// MFMA GEMM: y = A @ W^T with A (M, lda) bf16, never normalised here (as a
+// plain gemm_ring where that takes the shape).
 hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                 const EpiArgs& ea, hipStream_t st);
 // h = bf16(rms(x)) for M rows of length d (row strides ldx / ldh).

@@ -1327,7 +1327,8 @@ hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N
         gemm_big_fits(A, lda, M, N, K, ea))
       return gemm_big(A, lda, W, M, N, K, ea, st);
   }
-  if (gemm_ring_fits(epi, A, lda, W, M, N, K, ea)) return gemm_ring(epi, A, lda, W, M, N, K, ea, st);
+  if (gemm_ring_fits(epi, A, lda, W, M, N, K, ea))
+    return gemm_ring(epi, false, A, lda, W, M, N, K, ea, st);
   // what the ring kernel does not take (the top-k epilogue, a vocabulary that
   // is no multiple of 64): 64 x 128 tiles for at most 64 rows,
   // 128 x 128 below 512 rows, then 256 x 128

@@ -1,0 +1,49 @@
+"""Which tile of the ring GEMM a projection takes (host rule of gemm_ring.hip):
+a plain A never meets a tile that would normalise it, whatever the shape."""
+
+import ctypes
+import os
+
+import pytest
+
+from attention_nn_amd import _lib
+
+STORE, RELU2, RESID_ATTN, RESID_MLP, LOGITS, QKV, CE = range(7)
+
+
+@pytest.fixture(scope="module")
+def tile():
+    if not os.path.exists(_lib.LIB_PATH):
+        from attention_nn_amd.build import build
+        build()
+    f = ctypes.CDLL(_lib.LIB_PATH)._ZN3ann14gemm_ring_tileEibiii
+    f.argtypes, f.restype = [ctypes.c_int, ctypes.c_bool] + [ctypes.c_int] * 3, ctypes.c_int
+
+    def call(epi, rms, M, N, K):
+        t = f(epi, rms, M, N, K)
+        return t >> 16, t & 0xffff
+    return call
+
+
+def _takes_rms(epi, bm, bn):
+    """The small tiles of the qkv and fc epilogues form rms(A) in the product."""
+    return epi in (STORE, RELU2, QKV) and bm * bn <= 128 * 64
+
+
+@pytest.mark.parametrize("epi,cols", [(STORE, 3), (QKV, 3), (RELU2, 4), (RESID_ATTN, 1)])
+def test_plain_product_never_takes_a_normalising_tile(tile, epi, cols):
+    for d in (64, 128, 192, 512, 768, 1536):
+        if epi == QKV and d % 128:
+            continue
+        for M in (129, 130, 300, 777, 1027, 2048, 4096, 8192, 32768):
+            bm, bn = tile(epi, False, M, cols * d, d)
+            assert bm and cols * d % bn == 0 and not _takes_rms(epi, bm, bn), (d, M, bm, bn)
+            # the fastest tile of all where that one takes the rows as they are
+            any_bm, any_bn = tile(epi, True, M, cols * d, d)
+            assert _takes_rms(epi, any_bm, any_bn) or (any_bm, any_bn) == (bm, bn)
+
+
+def test_columns_of_64_alone_have_no_plain_tile(tile):
+    assert tile(STORE, False, 300, 320, 320) == (0, 0)
+    assert tile(STORE, True, 300, 320, 320)[1] == 64
+    assert tile(LOGITS, False, 300, 320, 320)[1] == 64
