@@ -362,9 +362,8 @@ static hipError_t attn_prefill_launch(hipStream_t st, const bf16_t* q, const bf1
                                       int T, int H, int max_ctx, int window, bool long_layer,
                                       float scale, float shift, int cus) {
   constexpr size_t lds = ap_lds_bytes<DH, BK, NS, KP>();
-  static const hipError_t attr =
-      hipFuncSetAttribute((const void*)k_attn_prefill<DH, BK, NS, KP>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  static PerDevice limit;
+  const hipError_t attr = lds_limit(limit, (const void*)k_attn_prefill<DH, BK, NS, KP>, lds);
   if (attr != hipSuccess) return attr;
   constexpr int BQ = 128 / KP;
   const dim3 grid((T + BQ - 1) / BQ, H, B);

@@ -875,15 +875,11 @@ size_t decode_persist_lds(int B, int d, int H, int Dh, int s_long) {
 template <int DH, int BM, int UD, int DM = 0, int HM = 0, int GR = 0>
 static hipError_t pd_launch(const PDParams& P, int G, size_t lds, bool coop, hipStream_t st) {
   const void* fn = (const void*)k_decode_persist<DH, BM, UD, DM, HM, GR>;
-  static bool attr = false;
-  if (!attr) {
-    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)PD_MAX_LDS);
-    if (e != hipSuccess) return e;
-    attr = true;
-  }
+  static PerDevice limit;
+  hipError_t e = lds_limit(limit, fn, PD_MAX_LDS);
+  if (e != hipSuccess) return e;
   int nb = 0;
-  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, PD_T, lds);
+  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, PD_T, lds);
   if (e != hipSuccess) return e;
   if (nb < 1) return hipErrorCooperativeLaunchTooLarge;
   PDParams a = P;

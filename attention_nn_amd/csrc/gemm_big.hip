@@ -293,8 +293,8 @@ bool gemm_big_fits(const bf16_t* A, int lda, int M, int N, int K, const EpiArgs&
 template <int BN>
 static hipError_t launch_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                              const EpiArgs& ea, hipStream_t st) {
-  static const hipError_t attr = hipFuncSetAttribute(
-      (const void*)k_gemm_big<BN>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BG_LDS);
+  static PerDevice limit;
+  const hipError_t attr = lds_limit(limit, (const void*)k_gemm_big<BN>, BG_LDS);
   if (attr != hipSuccess) return attr;
   const int nt = ((M + BG_BM - 1) / BG_BM) * (N / BN);
   const int grid = (nt + 7) / 8 * 8;

@@ -664,13 +664,20 @@ bool gemm_ring_rms(int epi, int M, int N, int K) {
 }
 
 hipError_t gemm_ring_prepare() {
-  static const bool ok = ring_attrs<EPI_STORE>() && ring_attrs<EPI_RELU2>() &&
-                         ring_attrs<EPI_RESID_ATTN>() && ring_attrs<EPI_RESID_MLP>() &&
-                         ring_attrs<EPI_LOGITS>() && ring_attr<EPI_CE, 128, 128, 2, 2, 2>() &&
-                         ring_attr<EPI_CE, 128, 192, 2, 2, 2>() && ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
-                         ring_attr<EPI_QKV, 64, 128, 3, 2, 2>() &&
-                         ring_attr<EPI_QKV, 192, 128, 2, 2, 2>();
-  return ok ? hipSuccess : hipErrorInvalidValue;
+  static PerDevice limits;
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  return (hipError_t)limits.once(dev, [] {
+    const bool ok = ring_attrs<EPI_STORE>() && ring_attrs<EPI_RELU2>() &&
+                    ring_attrs<EPI_RESID_ATTN>() && ring_attrs<EPI_RESID_MLP>() &&
+                    ring_attrs<EPI_LOGITS>() && ring_attr<EPI_CE, 128, 128, 2, 2, 2>() &&
+                    ring_attr<EPI_CE, 128, 192, 2, 2, 2>() &&
+                    ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
+                    ring_attr<EPI_QKV, 64, 128, 3, 2, 2>() &&
+                    ring_attr<EPI_QKV, 192, 128, 2, 2, 2>();
+    return (int)(ok ? hipSuccess : hipErrorInvalidValue);
+  });
 }
 
 hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* W, int M, int N,

@@ -3,8 +3,20 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "common.h"
+#include "per_device.h"
 
 namespace ann {
+
+// Allows a kernel `bytes` of dynamic LDS on the current device (more than 64 KB
+// has to be asked for); `state` is the kernel's own.
+inline hipError_t lds_limit(PerDevice& state, const void* kernel, size_t bytes) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  return (hipError_t)state.once(dev, [&] {
+    return (int)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  });
+}
 
 // Epilogue of a projection y = a @ W^T (W stored (N, K)):
 //   EPI_STORE       out = bf16(y)
@@ -135,7 +147,7 @@ int gemm_ring_tile(int epi, bool rms, int M, int N, int K);
 // not fit): ceil(N / columns) partial sums per row.
 int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                  const EpiArgs& ea);
-// One-time set-up (dynamic LDS limits), called by the entry points before
+// Dynamic LDS limits, once per device; called by the entry points before
 // anything they may capture into a graph.
 hipError_t gemm_ring_prepare();
 // The MLP's output projection (EPI_RESID_MLP) where its input is large: 256 x

@@ -857,9 +857,8 @@ hipError_t sample(const bf16_t* z, int ldz, int B, int Vs, const SampParams* sp,
 }
 
 hipError_t sample_prepare() {
-  static const hipError_t attr = hipFuncSetAttribute(
-      (const void*)k_sample_cand, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-  return attr;
+  static PerDevice limit;
+  return lds_limit(limit, (const void*)k_sample_cand, 128 * 1024);
 }
 
 hipError_t sample_cand(const uint32_t* cand, const uint32_t* cand_r, int nt, int holders, int B,
