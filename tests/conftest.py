@@ -18,3 +18,24 @@ def tiny_cfg():
     # the reference's own tiny self-test config (model.py:290-291)
     return GPTConfig(vocab_size=512, num_layers=2, num_heads=4, model_dim=64, seq_len=32,
                      window=16, long_layers=(1,))
+
+
+def _trace(fn):
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events()]
+
+
+@pytest.fixture(scope="session")
+def traced():
+    """traced(fn): the names of the kernels and runtime calls of one fn().
+    Skipped where the profiler sees no kernels (another tracer holds the device)."""
+    import torch
+    x = torch.zeros(1024, device="cuda")
+    if not any("elementwise" in n for n in _trace(lambda: x.add_(1))):
+        pytest.skip("no kernel trace on this machine")
+    return _trace

@@ -47,3 +47,20 @@ def test_columns_of_64_alone_have_no_plain_tile(tile):
     assert tile(STORE, False, 300, 320, 320) == (0, 0)
     assert tile(STORE, True, 300, 320, 320)[1] == 64
     assert tile(LOGITS, False, 300, 320, 320)[1] == 64
+
+
+def test_gpu_cases_reach_every_tile(tile):
+    """The row counts and widths of test_gpu_gemm_ring.py's cases, over the five
+    products of a forward.  (A plain-store qkv has 3 d columns of an odd multiple
+    of 64: never whole 128-column tiles.)"""
+    from test_gpu_gemm_ring import CASES
+    reached = set()
+    for d, _, V, B, T in CASES:
+        M, qkv = B * T, STORE if d % 128 else QKV
+        shapes = [(qkv, True, 3 * d, d), (RELU2, True, 4 * d, d), (RESID_ATTN, False, d, d),
+                  (RESID_MLP, False, d, 4 * d)] + ([(LOGITS, False, V, d)] if V % 64 == 0 else [])
+        reached |= {(epi, tile(epi, rms, M, N, K)) for epi, rms, N, K in shapes}
+    tiles = [(32, 64), (64, 64), (128, 64), (128, 128), (128, 192)]
+    want = {(epi, t) for epi in (STORE, RELU2, RESID_ATTN, RESID_MLP, LOGITS) for t in tiles}
+    want |= {(QKV, t) for t in [(64, 128), (128, 128), (192, 128)]}
+    assert want - reached == {(STORE, (128, 128))}

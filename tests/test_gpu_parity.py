@@ -964,46 +964,62 @@ def test_sample_api_slides_window_like_reference():
     assert got == ids[50:]
 
 
-# ---- the 256 x 256 prefill GEMM (gemm_big.hip) -------------------------------
+# ---- the 256-row GEMM of the MLP's output projection (gemm_big.hip) ----------
 
-def _big_cfg(dh):
-    return GPTConfig(vocab_size=4096, num_layers=2, num_heads=768 // dh if dh == 128 else 8,
-                     model_dim=768 if dh == 128 else 512, seq_len=512, window=100,
+def _big_cfg(dh, vocab=4096):
+    """d 768 (tiles of 192 columns at 8000 rows) or d 1024 (of 256)."""
+    return GPTConfig(vocab_size=vocab, num_layers=2, num_heads=6 if dh == 128 else 16,
+                     model_dim=768 if dh == 128 else 1024, seq_len=513, window=100,
                      long_layers=(1,))
 
 
+def _uses_big(names, cols):
+    return any(f"k_gemm_big<{cols}>" in n for n in names)
+
+
 @pytest.mark.parametrize("dh", [128, 64])
-def test_big_gemm_prefill_every_position(dh, monkeypatch):
-    """A prefill of 16 x 500 tokens (8000 rows: a ragged last 256-row tile)
-    puts the QKV (fused QK-norm / RoPE / cache epilogue), fc (relu^2) and, at
-    d = 768, the o / proj (residual mixes) projections on the 256 x 256 GEMM;
-    logits at every position against the oracle, and against the same
-    forward on the previous tiles (ANN_GEMM_BIG=0)."""
+def test_big_gemm_prefill_every_position(dh, monkeypatch, traced):
+    """A prefill of 16 x 500 tokens (8000 rows: a ragged last 256-row tile) with
+    the MLP's output projection (residual mix) on the 256-row GEMM
+    (ANN_GEMM_BIG=2: every shape it takes); logits at every position against
+    the oracle, and against the same forward on the ring kernel
+    (ANN_GEMM_BIG=0)."""
     cfg = _big_cfg(dh)
     p = perturb_lambdas(init_params(cfg, 71, dense=True))
     tok = np.random.default_rng(72).integers(0, cfg.vocab_size, (16, 500))
     print(f"case big gemm dh={dh} B=16 T=500", flush=True)
     eng = _engine(cfg, p, 16)
-    monkeypatch.setenv("ANN_GEMM_BIG", "2")    # every epilogue the kernel takes
+    monkeypatch.setenv("ANN_GEMM_BIG", "2")
     got = eng.forward_logits(tok).cpu()
-    monkeypatch.setenv("ANN_GEMM_BIG", "1")    # the routed ones (fc, o-proj)
-    routed = eng.forward_logits(tok).cpu()
+    assert _uses_big(traced(lambda: eng.forward_logits(tok)), 192 if dh == 128 else 256)
     monkeypatch.setenv("ANN_GEMM_BIG", "0")
-    old = eng.forward_logits(tok).cpu()
+    ring = eng.forward_logits(tok).cpu()
+    assert not any("k_gemm_big" in n for n in traced(lambda: eng.forward_logits(tok)))
     monkeypatch.delenv("ANN_GEMM_BIG")
     # same products in the same k order: equal up to the order of the K tiles'
     # accumulation inside an MFMA (measured bitwise equal)
-    assert (got - old).abs().max().item() < 2e-3
-    assert (routed - old).abs().max().item() < 2e-3
-    ref = R.logits(cfg, p, tok)
-    err = max((got - ref).abs().max().item(), (routed - ref).abs().max().item())
+    assert (got - ring).abs().max().item() < 2e-3
+    err = (got - R.logits(cfg, p, tok)).abs().max().item()
     assert err < LOGIT_TOL, err
 
 
-def test_big_gemm_training_forward():
-    """GPT.__call__ on 16 x 500 tokens (the body's projections on the 256 x
-    256 GEMM, the lm_head's CE epilogue on the previous tiles): per-row losses
-    against the oracle."""
+def test_big_gemm_routed_size(monkeypatch, traced):
+    """128 x 513 tokens at d 768 (an input of 403 MB, 257 tile rows) take the
+    256-row GEMM by themselves, on 256 columns; logits against the ring kernel's."""
+    cfg = _big_cfg(128, vocab=256)
+    p = perturb_lambdas(init_params(cfg, 75, dense=True))
+    tok = np.random.default_rng(76).integers(0, cfg.vocab_size, (128, 513))
+    print("case big gemm routed B=128 T=513", flush=True)
+    eng = _engine(cfg, p, 128)
+    got = eng.forward_logits(tok)
+    assert _uses_big(traced(lambda: eng.forward_logits(tok)), 256)
+    monkeypatch.setenv("ANN_GEMM_BIG", "0")
+    assert (got - eng.forward_logits(tok)).abs().max().item() < 2e-3
+
+
+def test_big_gemm_training_forward(monkeypatch, traced):
+    """GPT.__call__ on 16 x 500 tokens with the MLP's output projection on the
+    256-row GEMM: per-row losses against the oracle."""
     cfg = _big_cfg(128)
     p = perturb_lambdas(init_params(cfg, 73, dense=True))
     rng = np.random.default_rng(74)
@@ -1011,7 +1027,9 @@ def test_big_gemm_training_forward():
     tgt = rng.integers(0, cfg.vocab_size, (16, 500))
     print("case big gemm training forward", flush=True)
     eng = _engine(cfg, p, 16)
+    monkeypatch.setenv("ANN_GEMM_BIG", "2")
     mean, rows = eng.forward_loss(tok, tgt, rows=True)
+    assert _uses_big(traced(lambda: eng.forward_loss(tok, tgt)), 192)
     rm, rr = R.loss(cfg, p, tok, tgt, banded_bf16=True)
     assert (rows.cpu().double() - rr.double()).abs().max().item() < 1e-2
     assert abs(mean.item() - rm.item()) < 5e-4

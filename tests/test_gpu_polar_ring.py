@@ -6,8 +6,6 @@ A and B wherever the shorter side is whole tiles, aligned buffers or not."""
 import pytest
 import torch
 
-from torch.profiler import ProfilerActivity, profile
-
 import oracle.ref_optim as O
 
 pytestmark = pytest.mark.gpu
@@ -31,16 +29,6 @@ def test_polar_ring_matches_oracle(shape):
         assert torch.equal(G.polar_express(g[z:z + 1].cuda())[0], got[z])
 
 
-def _launches(fn, name):
-    """How many kernels of that name one call of fn launches."""
-    fn()
-    torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CUDA]) as prof:
-        fn()
-        torch.cuda.synchronize()
-    return sum(name in e.name for e in prof.events())
-
-
 def _polar_into(g, out):
     from attention_nn_amd import _lib
     from attention_nn_amd import optim as G
@@ -56,7 +44,7 @@ def _polar_into(g, out):
 @pytest.mark.parametrize("shape", [(2, 128, 192), (2, 320, 256), (1, 256, 320), (2, 384, 128),
                                    (1, 128, 384), (1, 192, 256)])
 @pytest.mark.parametrize("off_g,off_out", [(0, 0), (1, 0), (0, 1)])
-def test_polar_symmetric_products_take_half_their_tiles(shape, off_g, off_out):
+def test_polar_symmetric_products_take_half_their_tiles(shape, off_g, off_out, traced):
     """The five A and five B products on k_pe_ring where the shorter side is
     whole tiles; buffers at any element give the bits of aligned ones."""
     S, n = min(shape[1:]), torch.Size(shape).numel()
@@ -71,6 +59,7 @@ def test_polar_symmetric_products_take_half_their_tiles(shape, off_g, off_out):
     # which the general path only takes aligned
     skipped = 2 if off_out and shape[1] < shape[2] and max(shape[1:]) % 128 else 0
     half = S % 128 == 0
+    names = traced(lambda: _polar_into(g, out))
     for epi in (10, 7):
-        got = _launches(lambda: _polar_into(g, out), f"k_pe_ring<{epi}>")
+        got = sum(f"k_pe_ring<{epi}>" in n for n in names)
         assert got == (5 - (skipped if epi == 10 else 0) if half else 0)
