@@ -18,7 +18,8 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 // Grid (ceil(T/BQ), H, B), 512 threads: 8 waves in KP key parts of 8 / KP waves
 // x 16 queries (BQ = 128 / KP).  A ring stage holds KP tiles of BK keys, one
 // for each part; with KP > 1 the parts' sums are added through LDS at the end
-// (the fixed softmax shift leaves nothing to rescale).  K and V tiles stream
+// (the fixed softmax shift leaves nothing to rescale), so a sequence's fp32 sums
+// run in an order that depends on the grid it is part of.  K and V tiles stream
 // through a ring of NS LDS stages: each tile is loaded straight into LDS
 // (global_load_lds_dwordx4, 1 KB per wave instruction, no register staging)
 // NS - 1 stages ahead of its use; one barrier per stage.  LDS

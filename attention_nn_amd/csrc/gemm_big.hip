@@ -261,9 +261,12 @@ int device_cus() {
 
 // Whether an (M, N) = (rows, d) product over K comes here instead of
 // k_gemm_ring: where A is 384 MB or more, past the memory-side cache.  Ring
-// against here, in us: d 768 (K 3072) at 32768 rows 137 / 150, at 65536 300 /
-// 284, at 122880 557 / 536; d 1536 (K 6144) at 16384 rows 272 / 276, at 32768
-// 550 / 509, at 65536 1076 / 989, at 131072 2136 / 1975.
+// against here, in us, behind the fc projection that has just written A (in
+// brackets repeated by itself): d 768 (K 3072) at 16384 rows 65 / 70 (67 / 67), at
+// 32768 164 / 161 (131 / 138: A stays in the memory-side cache), at 65536 296 /
+// 268 (300 / 272), at 122880 555 / 523 (549 / 519); d 1536 (K 6144) at 8192 rows
+// 129 / 130 (127 / 125), at 16384 285 / 273 (258 / 251), at 32768 552 / 494 (548
+// / 489), at 65536 1078 / 1000 (1076 / 979), at 122880 2004 / 2058 (2001 / 1919).
 bool gemm_big_routes(int M, int K) { return (long long)M * K >= 192LL << 20; }
 
 // Tile width for an M x N output: 256 or 192 columns, whichever needs fewer

@@ -4,19 +4,20 @@
 // (global_load_lds_dwordx4, no register staging), one barrier per K tile; the
 // output tile is chosen by the shape (ring_pick).
 //
-// What bounds it.  A lone work-group and a full CU take the same time per K
-// tile of a 64 x 64 or 128 x 64 tile, 0.2 and 0.31 us: 16 and 24 KB through the
-// CU's load path, about 80 GB/s per CU (38 of its 64 bytes per clock).  So a
-// shape that leaves CUs idle wants small tiles on all of them, and a shape
-// that fills them wants large tiles, which move fewer bytes per flop: 128 x
-// 128 takes 0.51 us and 128 x 192 0.64 us per K tile, where the MFMAs alone
-// take 0.31 and 0.46 (1.75 PFLOP/s, the form's measured ceiling).  Two
-// work-groups share a CU at every tile: their barriers fall apart in time, so
-// one reads LDS and waits while the other multiplies, and one's epilogue runs
-// under the other's main loop.  One work-group of eight waves with the same
-// tiles (256 x 128, two or three stages) is slower for that reason (proj of
-// 32768 rows, d 768: 160 against 147 us), as are K tiles of 32 (half cache
-// lines: 171) and v_mfma_f32_32x32x16 (164 against 133 at 128 x 128).
+// What bounds it.  Time per K tile (slope over K, residual epilogue) at 32 x 64,
+// 64 x 64, 128 x 64, 128 x 128 and 128 x 192: 0.17, 0.24, 0.36, 0.60 and 0.73 us
+// with one work-group on each CU, 0.30, 0.38, 0.56, 0.86 and 1.20 for two that
+// share one -- 16 and 24 KB a work-group of the 64- and 128 x 64 tiles through
+// the CU's load path, about 85 GB/s per CU.  So a shape that leaves CUs idle wants
+// small tiles on all of them, and a shape that fills them wants large tiles,
+// which move fewer bytes per flop: 0.43 and 0.60 us a work-group at 128 x 128 and
+// 128 x 192, where the MFMAs alone take 0.31 and 0.46 (1.75 PFLOP/s, the form's
+// measured ceiling).  Two work-groups share a CU at every tile: their barriers
+// fall apart in time, so one reads LDS and waits while the other multiplies, and
+// one's epilogue runs under the other's main loop.  One work-group of eight waves
+// with the same tiles (256 x 128, two or three stages) is slower for that reason
+// (proj of 32768 rows, d 768: by 9%), as are K tiles of 32 (half cache lines: 16%)
+// and v_mfma_f32_32x32x16 (23% at 128 x 128).
 #include <type_traits>
 #include "common.h"
 #include "epilogue.h"
@@ -398,8 +399,11 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
                                                       softcap(lo_f(y.w)), softcap(hi_f(y.w)));
         }
       } else if constexpr (EPI == EPI_RELU2 && BN == 192) {
-        // a large fc output, read back once by the next projection: past the
-        // caches (fc of 32768 rows, d 768: 163 -> 157 us at 128 x 128)
+        // The tile of the large fc outputs, which the next projection reads back
+        // once: past the caches.  Plain stores against these, whole calls: 16 x
+        // 7680 tokens and 32 steps 44.43 / 44.21 ms, d 1536 128 x 1024 tokens and
+        // 24 steps 36.19 / 36.08; prompts of 8 x 512 tokens 1413 / 1386 us, but of
+        // 2 x 962 992 / 1004, 16 x 512 2261 / 2273, 32 x 512 3627 / 3637.
         __builtin_nontemporal_store(__builtin_bit_cast(rg_u32x4, y),
                                     (rg_u32x4*)(ea.out + (size_t)m * ea.ldo + n));
       } else {
@@ -573,8 +577,9 @@ bool ring_attrs() {
 }
 
 // The tiles, with the time per K tile of a work-group alone on its CU and of
-// one of two that share it, and what a launch takes besides, in ns (measured
-// on the o / proj / fc shapes of d 512, 768 and 1536).
+// one of two that share it, and what a launch takes besides, in ns: fitted on the
+// o / proj / fc shapes of d 512, 768 and 1536 (within 13% of the slopes above,
+// whose epilogue is one of several).
 struct RingTile {
   int bm, bn;
   int alone, shared, fixed;
@@ -582,7 +587,14 @@ struct RingTile {
 constexpr RingTile RING_TILES[] = {
     {32, 64, 150, 145, 2800},   {64, 64, 207, 195, 2900},   {128, 64, 340, 290, 3600},
     {128, 128, 590, 470, 4600}, {128, 192, 780, 660, 5000},
-    // QKV only (a 128-column tile holds whole heads)
+    // QKV only (a 128-column tile holds whole heads).  Its epilogue costs 2 to 3 us
+    // a work-group at every tile, which leaves the order of the three to the
+    // products: the times of the same tiles transposed, measured as a rule with the
+    // three tiles at 19 row counts from 200 to 131072 of d 128, 256, 512, 768 and
+    // 1536 (2 us added to the tiles whose x a launch normalises): the fastest or
+    // within 5% of it at 92 of the 95, 10% off at the worst.  64 x 128 / 128 x 128 /
+    // 192 x 128, d 768: 777 rows 10.4 / 11.9 / 15.6 us, 4096 29.7 / 26.2 / 24.4,
+    // 16384 101 / 75 / 77, 131072 811 / 603 / 555.
     {64, 128, 340, 290, 3600},  {192, 128, 780, 660, 5000}};
 constexpr int RING_N = 5, RING_QKV_N = 7;
 
@@ -597,9 +609,9 @@ static bool ring_has(const RingTile& t, int i, int epi, bool plain) {
 }
 
 // The tile that is done first: the CU with the most work-groups takes them in
-// pairs (two are resident).  Measured against every tile at 130 .. 32768 rows
-// of d 512, 768 and 1536: within 5% of the best one at most shapes, 15% at
-// the worst.  -1 where no tile divides N (of any A: N is a multiple of 64, of
+// pairs (two are resident).  Measured against every tile of o, proj and fc at 130
+// .. 32768 rows of d 512, 768 and 1536: within 5% of the best one at most
+// shapes, 15% at the worst (QKV: at RING_TILES).  -1 where no tile divides N (of any A: N is a multiple of 64, of
 // 128 for QKV; plain qkv and fc: of 128 or 192).
 static int ring_pick(int epi, bool plain, int M, int N, int K) {
   static const int cus = device_cus();

@@ -247,8 +247,9 @@ hipError_t attn_decode(const bf16_t* qkv, bf16_t* kc, bf16_t* vc, const int32_t*
 // The decode step's RMS + qkv projection (x (B, d) against wqkv (3d, d)) and
 // the attention above in one launch: q, k, v handed over as tagged words in
 // xt (B x 3d/2 words; `tag` larger than any earlier launch's on that buffer).
-// Shapes it takes: 4..64 rows (the skinny GEMM's; fewer run on the GEMV), Dh 128,
-// d a multiple of 128 up to 768.
+// Shapes it takes: 4..64 rows, Dh 128, d a multiple of 128 up to 768.  From 4:
+// fewer rows run in the persistent step (155M: 4 too); where that is off, 1 and 2
+// rows are the GEMV's and 3 keep their replayed graph.
 constexpr bool qkv_attn_fits(int B, int d, int Dh) {
   return B >= 4 && B <= 64 && Dh == 128 && d % 128 == 0 && d <= 768;
 }

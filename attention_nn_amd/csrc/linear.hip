@@ -1155,8 +1155,8 @@ hipError_t gemm_skinny(int epi, bool rms, const bf16_t* A, int lda, const bf16_t
     const int xd = T == 2 && kw % 4 == 0 && (kw / 4) % 3 == 0 ? 3 : 1;
     // The o / proj projections on 16 x 16 tiles: eight waves instead of four
     // halve each wave's chain of rounds where their larger LDS costs no
-    // resident work-group: short chains (K <= 768: 51 KB), or at most one work-
-    // group per CU (102 KB).  155M decode step of 7 / 16 / 64 / 80 rows 322 ->
+    // resident work-group: short chains (K <= 768: 52 KB), or at most one work-
+    // group per CU (100 KB).  155M decode step of 7 / 16 / 64 / 80 rows 322 ->
     // 310, 337 -> 325, 470 -> 459, 552 -> 540 us, d 1536 at 8 rows (three
     // layers) 179 -> 169; proj with more work-groups than CUs is slower (100
     // rows 596 -> 615).  16 waves: within 1% of eight.

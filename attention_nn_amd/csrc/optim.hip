@@ -11,8 +11,9 @@
 //    every product is an "NT" GEMM: x x^T directly, A A because A is symmetric,
 //    B x through one transpose of x per iteration (x B for tall matrices, B
 //    symmetric); their A and B still run on the ring kernel where the shorter
-//    side is whole tiles (22 x 768 x 2880: 1839 -> 1305 us).  The combinations b A + c A^2 and a x + B x run in the
-//    epilogues with the eager rounding of each op.
+//    side is whole tiles (22 x 768 x 2880: 1839 -> 1305 us).  The combinations
+//    b A + c A^2 and a x + B x run in the epilogues with the eager rounding of
+//    each op.
 //  * NorMuon (muon.py:47-63): mean of squares along the reduced axis, one
 //    work-group per matrix for the norms and the second-moment update, then
 //    the broadcast scale.
