@@ -2,10 +2,10 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-secondary] [--no-cpu]
 
-Workload: 155M model (d768, 11 layers, 6 heads x
-128, long layers {4,10}, window 384, vocab 50304), random-init bf16 weights
-(model.py distributions, Wo/proj drawn dense), batch 1, 32-token random
-prompt, greedy decode to context 1024.  A "step" is one whole generation of
+Workload: 155M model (d768, 11 layers, 6 heads x 128, long layers {4,10},
+window 384, vocab 50304), random-init bf16 weights (model.py distributions,
+Wo/proj drawn dense), batch 1, 32-token random prompt, greedy decode to
+context 1024.  A "step" is one whole generation of
 that workload: the prefill of the 32-token prompt (which samples the first
 token) and 991 decode steps, 992 generated tokens at positions 32..1023.  K
 steps are timed between two device synchronisations with HIP events on the
@@ -30,10 +30,9 @@ non-zero if one did.
 
 secondary: the same batch-1 generation sampled at sample.py's defaults
 (T = 0.8, top-k 50; median of 3); each of the following the median of 5
-repetitions: batch-64 decode (configs[2]:
-512-token prompts, temperature 0.8, top-k 50) against HBM and its prefill
-against the bf16 MFMA peak; the training forward; one optimizer step;
-configs[3] (B=16 at context 8192) and configs[4] (d1536, B=128).
+repetitions: batch-64 decode (512-token prompts, temperature 0.8, top-k 50)
+against HBM and its prefill against the bf16 MFMA peak; the training forward; one optimizer step;
+the 155M at B=16 and context 8192, and the d1536 model at B=128.
 
 cpu_baseline: the CPU oracle (PyTorch restatement of model.py's forward)
 with sample.py's semantics -- a full forward over the whole context for every
@@ -274,7 +273,7 @@ def decode_section(cfg, params, B, P, S, temp, k, seed, eng=None):
 
 
 def secondary_b64(cfg, params):
-    """configs[2]: B=64, 512-token prompts: prefill vs MFMA, 512 decode steps
+    """B=64, 512-token prompts: prefill vs MFMA, 512 decode steps
     at T=0.8 / top-k 50 vs HBM; and the training forward on the same tokens."""
     import torch
     from attention_nn_amd.engine import Engine
@@ -353,7 +352,7 @@ def secondary_optim(cfg, params):
 
 
 def extra_config(name):
-    """prefill then decode, medians of REPS."""
+    """One (B, prompt, steps) configuration: prefill then decode, medians of REPS."""
     from attention_nn_amd.config import cfg_155m, cfg_834m
     from attention_nn_amd.weights import init_params
     if name == "cfg4":

@@ -7,7 +7,7 @@ Metal kernels it calls (``metal_kernels.py:37-47`` relu2,
 training forward's loss ``GPT.__call__`` (``model.py:180-221``) with its
 fused softcapped cross-entropy (``metal_kernels.py:153-193``).  Only ``tests/``,
 ``__graft_entry__.smoke()`` and ``bench.py``'s cpu_baseline leg may import
-this module, and only as the checker or the timed CPU baseline; the product
+this module, and only as the oracle or the timed CPU baseline; the product
 path (``attention_nn_amd``) never calls it.
 
 Rounding model ("fp32 masters, bf16 compute", eager MLX):
