@@ -1,6 +1,6 @@
 // The MLP's output projection x = r1 x + p1 (h @ W^T) (W stored (N, K) bf16)
-// where h is larger than the memory-side cache (gemm_big_routes has the
-// measurements against k_gemm_ring): 256 x 256 (or 256 x 192) output tiles of
+// where its tiles fill the CUs (gemm_big_routes has the measurements against
+// k_gemm_ring): 256 x 256 (or 256 x 192) output tiles of
 // four waves of 128 x 128 (128 x 96), one work-group (one wave per SIMD) per
 // CU, v_mfma_f32_16x16x32_bf16 -- the tile that moves the fewest bytes per
 // flop.
@@ -259,16 +259,6 @@ int device_cus() {
   return cus;
 }
 
-// Whether an (M, N) = (rows, d) product over K comes here instead of
-// k_gemm_ring: where A is 384 MB or more, past the memory-side cache.  Ring
-// against here, in us, behind the fc projection that has just written A (in
-// brackets repeated by itself): d 768 (K 3072) at 16384 rows 65 / 70 (67 / 67), at
-// 32768 164 / 161 (131 / 138: A stays in the memory-side cache), at 65536 296 /
-// 268 (300 / 272), at 122880 555 / 523 (549 / 519); d 1536 (K 6144) at 8192 rows
-// 129 / 130 (127 / 125), at 16384 285 / 273 (258 / 251), at 32768 552 / 494 (548
-// / 489), at 65536 1078 / 1000 (1076 / 979), at 122880 2004 / 2058 (2001 / 1919).
-bool gemm_big_routes(int M, int K) { return (long long)M * K >= 192LL << 20; }
-
 // Tile width for an M x N output: 256 or 192 columns, whichever needs fewer
 // CU-rounds times columns (one work-group per CU), a 192-column tile counted
 // 15% dearer per column (less reuse of each A tile: 480 x 16 tiles of 192
@@ -280,6 +270,32 @@ static int big_bn(int M, int N) {
   const long long ntm = (M + BG_BM - 1) / BG_BM;
   auto rounds = [&](int bn) { return (ntm * (N / bn) + cus - 1) / cus; };
   return rounds(192) * 192 * 115 < rounds(256) * 256 * 100 ? 192 : 256;
+}
+
+// Whether an (M, N) = (rows, d) product over K comes here instead of
+// k_gemm_ring.  Here a full round of the CUs takes 1.53 us per K tile and 17 us
+// besides at 256 columns, 1.21 and 17 at 192, and a round that is not full hardly
+// less; the ring takes 1.2 times its rule's figure behind the fc projection that
+// has just written A (those are of a launch repeated by itself).  So a shape that
+// fills its rounds comes here, and most of what is past the memory-side cache,
+// where the ring's narrower tiles read A more often.  Measured behind the fc, ring
+// / here, us: d 512 (K 2048) at 16384 rows 35 / 59, 40960 90 / 122, 65536 167 /
+// 127; d 768 at 8192 rows 52 / 65, 16384 77 / 73, 19200 108 / 90, 32768 161 /
+// 149, 65536 328 / 298; d 1024 at 16384 124 / 117, 19200 155 / 213, 32768 323 /
+// 261; d 1536 at 4096 98 / 121, 10240 193 / 164, 16384 285 / 261, 32768 569 /
+// 512; d 2048 at 8192 233 / 213, 10240 322 / 374, 16384 544 / 472.  Over 99 shapes
+// of d 256 .. 2048 the choice loses 0.7% on the faster one in the mean and 11% at
+// the worst (12288 rows, d 1024: 97 / 108).
+bool gemm_big_routes(int M, int N, int K) {
+  static const int cus = device_cus();
+  const int bn = big_bn(M, N);
+  if (N % bn) return false;
+  const long long ring = gemm_ring_ns(EPI_RESID_MLP, false, M, N, K);
+  if (ring < 0) return true;
+  const long long tiles = (long long)((M + BG_BM - 1) / BG_BM) * (N / bn);
+  const long long ns = (tiles + cus - 1) / cus *
+                       ((long long)(K / BG_BK) * (bn == 256 ? 1530 : 1210) + 17000);
+  return ns * 5 < ring * 6;
 }
 
 // Whether gemm_big can take (M, N, K): whole 256- or 192-column tiles, 64-deep

@@ -613,7 +613,7 @@ static bool ring_has(const RingTile& t, int i, int epi, bool plain) {
 // .. 32768 rows of d 512, 768 and 1536: within 5% of the best one at most
 // shapes, 15% at the worst (QKV: at RING_TILES).  -1 where no tile divides N (of any A: N is a multiple of 64, of
 // 128 for QKV; plain qkv and fc: of 128 or 192).
-static int ring_pick(int epi, bool plain, int M, int N, int K) {
+static int ring_pick(int epi, bool plain, int M, int N, int K, long long* est_ns = nullptr) {
   static const int cus = device_cus();
   int best = -1;
   long long best_ns = 0;
@@ -628,7 +628,13 @@ static int ring_pick(int epi, bool plain, int M, int N, int K) {
       best_ns = ns;
     }
   }
+  if (est_ns) *est_ns = best_ns;
   return best;
+}
+
+long long gemm_ring_ns(int epi, bool rms, int M, int N, int K) {
+  long long ns = 0;
+  return ring_pick(epi, !rms, M, N, K, &ns) < 0 ? -1 : ns;
 }
 
 int gemm_ring_tile(int epi, bool rms, int M, int N, int K) {

@@ -141,8 +141,10 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
 bool gemm_ring_rms(int epi, int M, int N, int K);
 hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* W, int M, int N,
                      int K, const EpiArgs& ea, hipStream_t st);
-// The tile it takes: rows << 16 | columns, 0 where there is none.
+// The tile it takes (rows << 16 | columns, 0 where there is none) and what its
+// rule puts the launch at (-1 where there is none).
 int gemm_ring_tile(int epi, bool rms, int M, int N, int K);
+long long gemm_ring_ns(int epi, bool rms, int M, int N, int K);
 // Columns of gemm_ring's EPI_CE tiles (of gemm()'s, 128, where the ring does
 // not fit): ceil(N / columns) partial sums per row.
 int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
@@ -150,11 +152,11 @@ int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
 // Dynamic LDS limits, once per device; called by the entry points before
 // anything they may capture into a graph.
 hipError_t gemm_ring_prepare();
-// The MLP's output projection (EPI_RESID_MLP) where its input is large: 256 x
-// 256 tiles, one work-group per CU, AGPR accumulators.  gemm_big_fits says
+// The MLP's output projection (EPI_RESID_MLP) where its tiles fill the CUs: 256
+// x 256 or 192, one work-group per CU, AGPR accumulators.  gemm_big_fits says
 // whether a shape can go there, gemm_big_routes whether it is the faster one.
 bool gemm_big_fits(const bf16_t* A, int lda, int M, int N, int K, const EpiArgs& ea);
-bool gemm_big_routes(int M, int K);
+bool gemm_big_routes(int M, int N, int K);
 hipError_t gemm_big(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                     const EpiArgs& ea, hipStream_t st);
 // Compute units of the current device (256 where the query fails).

@@ -1316,14 +1316,14 @@ hipError_t gemm_decode64(int epi, const bf16_t* A, int lda, const bf16_t* W, int
 hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                 const EpiArgs& ea, hipStream_t st) {
   if (K % GM_BK != 0 || M <= 0 || N <= 0) return hipErrorInvalidValue;
-  // the MLP's output projection of a large input: the 256 x 256 one-work-
-  // group-per-CU kernel (gemm_big.hip).  ANN_GEMM_BIG=0 keeps it on the ring
+  // the MLP's output projection of a large input: the 256-row one-work-group-
+  // per-CU kernel where it is the faster one (gemm_big.hip).  ANN_GEMM_BIG=0 keeps it on the ring
   // kernel, ANN_GEMM_BIG=2 sends every shape it takes there (read at every
   // call)
   if (epi == EPI_RESID_MLP) {
     const char* big_env = getenv("ANN_GEMM_BIG");
     const int big_mode = big_env ? atoi(big_env) : 1;
-    if (big_mode != 0 && (big_mode == 2 || gemm_big_routes(M, K)) &&
+    if (big_mode != 0 && (big_mode == 2 || gemm_big_routes(M, N, K)) &&
         gemm_big_fits(A, lda, M, N, K, ea))
       return gemm_big(A, lda, W, M, N, K, ea, st);
   }

@@ -1,5 +1,6 @@
-"""Which tile of the ring GEMM a projection takes (host rule of gemm_ring.hip):
-a plain A never meets a tile that would normalise it, whatever the shape."""
+"""Which kernel and tile a prompt's projection takes (host rules of
+gemm_ring.hip and gemm_big.hip): a plain A never meets a tile that would
+normalise it, and the MLP's output projection takes the faster kernel."""
 
 import ctypes
 import os
@@ -64,3 +65,18 @@ def test_gpu_cases_reach_every_tile(tile):
     want = {(epi, t) for epi in (STORE, RELU2, RESID_ATTN, RESID_MLP, LOGITS) for t in tiles}
     want |= {(QKV, t) for t in [(64, 128), (128, 128), (192, 128)]}
     assert want - reached == {(STORE, (128, 128))}
+
+
+# us behind the fc projection that writes A, on 256 CUs: the ring, the 256-row kernel
+@pytest.mark.parametrize("d,M,ring,big", [
+    (512, 16384, 35, 59), (512, 40960, 90, 122), (512, 65536, 167, 127), (512, 98304, 249, 195),
+    (768, 8192, 52, 65), (768, 10240, 52, 66), (768, 19200, 108, 90), (768, 65536, 328, 298),
+    (1024, 8192, 62, 104), (1024, 19200, 155, 213), (1024, 28000, 277, 231),
+    (1024, 32768, 323, 261), (1024, 40960, 365, 324), (1280, 14000, 181, 237),
+    (1280, 24576, 360, 301), (1280, 65536, 897, 718), (1536, 4096, 98, 121),
+    (1536, 10240, 193, 164), (1536, 16384, 285, 261), (1536, 32768, 569, 512),
+    (2048, 8192, 233, 213), (2048, 10240, 322, 374), (2048, 16384, 544, 472)])
+def test_mlp_output_projection_takes_the_faster_kernel(tile, d, M, ring, big):
+    f = ctypes.CDLL(_lib.LIB_PATH)._ZN3ann15gemm_big_routesEiii
+    f.restype = ctypes.c_bool
+    assert f(M, d, 4 * d) == (big < ring)

@@ -1004,13 +1004,13 @@ def test_big_gemm_prefill_every_position(dh, monkeypatch, traced):
 
 
 def test_big_gemm_routed_size(monkeypatch, traced):
-    """128 x 513 tokens at d 768 (an input of 403 MB, 257 tile rows) take the
-    256-row GEMM by themselves, on 256 columns; logits against the ring kernel's."""
+    """127 x 513 tokens at d 768 (255 tile rows) take the 256-row GEMM by
+    themselves, on 256 columns; logits against the ring kernel's."""
     cfg = _big_cfg(128, vocab=256)
     p = perturb_lambdas(init_params(cfg, 75, dense=True))
-    tok = np.random.default_rng(76).integers(0, cfg.vocab_size, (128, 513))
-    print("case big gemm routed B=128 T=513", flush=True)
-    eng = _engine(cfg, p, 128)
+    tok = np.random.default_rng(76).integers(0, cfg.vocab_size, (127, 513))
+    print("case big gemm routed B=127 T=513", flush=True)
+    eng = _engine(cfg, p, 127)
     got = eng.forward_logits(tok)
     assert _uses_big(traced(lambda: eng.forward_logits(tok)), 256)
     monkeypatch.setenv("ANN_GEMM_BIG", "0")
