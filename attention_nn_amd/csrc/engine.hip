@@ -1013,8 +1013,7 @@ int ann_forward_loss(ann_ctx* c, const int32_t* tokens, const int32_t* targets, 
             c->c.d, M, c->c.V, c->c.d, ec, st);
   if (rc) return rc;
   float* rows = row_loss ? row_loss : c->sp<float>(c->sl.ce_rows);
-  const int cols = gemm_ce_cols(c->sp<bf16_t>(c->sl.hn), c->c.d, c->wptr(c->wl.head), M, c->c.V,
-                                c->c.d, ec);
+  const int cols = gemm_ce_cols(M, c->c.V, c->c.d);
   HIPCHK(ce_finalize(ec.ce_part, M, (c->c.V + cols - 1) / cols, ec.ce_tz, M, rows, loss, st));
   HIPCHK(advance_pos(pos, B, T, st));
   c->len = T;

@@ -221,7 +221,7 @@ __device__ __forceinline__ void ring_product(const bf16_t* A, int lda, const bf1
 }
 
 // WR x WC waves.  gm: tile rows per group of the tile order.
-template <int EPI, int BM, int BN, int NS, int WR, int WC>
+template <int EPI, int BM, int BN, int NS, int WR, int WC, bool RAG = false>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_ring(
     const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int M, int N, int K,
     int gm, EpiArgs ea) {
@@ -305,7 +305,9 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
     // in-lane over the wave's N blocks, then over the four lane groups, then
     // the column parts through LDS, always in the same order.  Hardware exp2
     // and reciprocal: the IEEE expf and division cost ~35 VALU instructions
-    // per logit.
+    // per logit.  RAG: the vocabulary ends inside the last tile, columns past it
+    // add nothing (an instance of its own: a uniform branch between the two costs
+    // the whole tiles 5%).
     float* red = (float*)rg_smem;
     float rs[MT];
 #pragma unroll
@@ -319,7 +321,8 @@ __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2)
         for (int r = 0; r < 4; ++r) {
           const int n = n0 + wn * WN + j * 16 + kg * 4 + r;
           const float zc = softcap_fast(rbf(acc[j][i][r]));
-          sum += __builtin_amdgcn_exp2f(zc * 1.4426950408889634f);
+          const float e = __builtin_amdgcn_exp2f(zc * 1.4426950408889634f);
+          sum += !RAG || n < N ? e : 0.f;
           if (n == tg) ea.ce_tz[m] = zc;
         }
       sum += __shfl_xor(sum, 16, 64);
@@ -552,20 +555,20 @@ hipError_t pe_ring(int epi, const bf16_t* A, int lda, long long sA, const bf16_t
 
 namespace {
 
-template <int EPI, int BM, int BN, int NS, int WR, int WC>
+template <int EPI, int BM, int BN, int NS, int WR, int WC, bool RAG = false>
 hipError_t launch_ring(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                        const EpiArgs& ea, hipStream_t st) {
-  if (N % BN) return hipErrorInvalidValue;
-  const dim3 grid(N / BN, (M + BM - 1) / BM);
-  hipLaunchKernelGGL((k_gemm_ring<EPI, BM, BN, NS, WR, WC>), grid, dim3(64 * WR * WC),
+  if (!RAG && N % BN) return hipErrorInvalidValue;
+  const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+  hipLaunchKernelGGL((k_gemm_ring<EPI, BM, BN, NS, WR, WC, RAG>), grid, dim3(64 * WR * WC),
                      (rg_lds_bytes<BM, BN, NS>()), st, A, lda, W, M, N, K, 4, ea);
   return hipGetLastError();
 }
 
 // dynamic LDS beyond 64 KB has to be asked for
-template <int EPI, int BM, int BN, int NS, int WR, int WC>
+template <int EPI, int BM, int BN, int NS, int WR, int WC, bool RAG = false>
 bool ring_attr() {
-  return hipFuncSetAttribute((const void*)k_gemm_ring<EPI, BM, BN, NS, WR, WC>,
+  return hipFuncSetAttribute((const void*)k_gemm_ring<EPI, BM, BN, NS, WR, WC, RAG>,
                              hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)rg_lds_bytes<BM, BN, NS>()) == hipSuccess;
 }
@@ -611,16 +614,17 @@ static bool ring_has(const RingTile& t, int i, int epi, bool plain) {
 // The tile that is done first: the CU with the most work-groups takes them in
 // pairs (two are resident).  Measured against every tile of o, proj and fc at 130
 // .. 32768 rows of d 512, 768 and 1536: within 5% of the best one at most
-// shapes, 15% at the worst (QKV: at RING_TILES).  -1 where no tile divides N (of any A: N is a multiple of 64, of
-// 128 for QKV; plain qkv and fc: of 128 or 192).
+// shapes, 15% at the worst (QKV: at RING_TILES).  -1 where no tile divides N (of
+// any A: N is a multiple of 64, of 128 for QKV; plain qkv and fc: of 128 or 192;
+// the loss takes every N).
 static int ring_pick(int epi, bool plain, int M, int N, int K, long long* est_ns = nullptr) {
   static const int cus = device_cus();
   int best = -1;
   long long best_ns = 0;
   for (int i = 0; i < RING_QKV_N; ++i) {
     const RingTile& t = RING_TILES[i];
-    if (!ring_has(t, i, epi, plain) || N % t.bn) continue;
-    const long long wgs = (long long)((M + t.bm - 1) / t.bm) * (N / t.bn);
+    if (!ring_has(t, i, epi, plain) || (epi != EPI_CE && N % t.bn)) continue;
+    const long long wgs = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const long long n = (wgs + cus - 1) / cus;
     const long long ns = K / RG_BK * (n / 2 * 2 * t.shared + n % 2 * t.alone) + t.fixed;
     if (best < 0 || ns < best_ns) {
@@ -643,10 +647,10 @@ int gemm_ring_tile(int epi, bool rms, int M, int N, int K) {
 }
 
 // Rows of A and of the epilogue's operands in 16-byte words, whole 64-column
-// tiles.
+// tiles (the loss: any vocabulary).
 bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
                     const EpiArgs& ea) {
-  if (M < 1 || N < 64 || N % 64 || K < RG_BK || K % RG_BK || lda % 8 ||
+  if (M < 1 || N < 1 || (epi != EPI_CE && N % 64) || K < RG_BK || K % RG_BK || lda % 8 ||
       (((uintptr_t)A | (uintptr_t)W) & 15))
     return false;
   switch (epi) {
@@ -661,7 +665,7 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
     case EPI_QKV:
       return gemm_qkv_fits(M, N, K, ea);
     case EPI_CE:
-      return (N % 128 == 0 || N % 192 == 0) && ea.ce_part && ea.ce_tz && ea.tgt && ea.ldz >= M;
+      return ea.ce_part && ea.ce_tz && ea.tgt && ea.ldz >= M;
     case EPI_LOGITS:
       return !ea.amax && ea.ldz % 8 == 0 && (((uintptr_t)ea.z | (uintptr_t)ea.logits) & 15) == 0;
     default:
@@ -669,12 +673,7 @@ bool gemm_ring_fits(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, i
   }
 }
 
-int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                 const EpiArgs& ea) {
-  return gemm_ring_fits(EPI_CE, A, lda, W, M, N, K, ea)
-             ? RING_TILES[ring_pick(EPI_CE, true, M, N, K)].bn
-             : 128;
-}
+int gemm_ce_cols(int M, int N, int K) { return RING_TILES[ring_pick(EPI_CE, true, M, N, K)].bn; }
 
 bool gemm_ring_rms(int epi, int M, int N, int K) {
   const int i = ring_pick(epi, false, M, N, K);
@@ -691,6 +690,8 @@ hipError_t gemm_ring_prepare() {
                     ring_attrs<EPI_RESID_ATTN>() && ring_attrs<EPI_RESID_MLP>() &&
                     ring_attrs<EPI_LOGITS>() && ring_attr<EPI_CE, 128, 128, 2, 2, 2>() &&
                     ring_attr<EPI_CE, 128, 192, 2, 2, 2>() &&
+                    ring_attr<EPI_CE, 128, 128, 2, 2, 2, true>() &&
+                    ring_attr<EPI_CE, 128, 192, 2, 2, 2, true>() &&
                     ring_attr<EPI_QKV, 128, 128, 2, 2, 2>() &&
                     ring_attr<EPI_QKV, 64, 128, 3, 2, 2>() &&
                     ring_attr<EPI_QKV, 192, 128, 2, 2, 2>();
@@ -723,6 +724,10 @@ hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* 
     case EPI_RESID_MLP: RING(EPI_RESID_MLP)
     case EPI_LOGITS: RING(EPI_LOGITS)
     case EPI_CE:
+      if (tile >= 0 && N % RING_TILES[tile].bn) {
+        if (tile == 3) return launch_ring<EPI_CE, 128, 128, 2, 2, 2, true>(A, lda, W, M, N, K, ea, st);
+        return launch_ring<EPI_CE, 128, 192, 2, 2, 2, true>(A, lda, W, M, N, K, ea, st);
+      }
       switch (tile) {
         RING_TILE(EPI_CE, 3, 128, 128, 2, 2, 2)
         RING_TILE(EPI_CE, 4, 128, 192, 2, 2, 2)

@@ -145,10 +145,8 @@ hipError_t gemm_ring(int epi, bool rms, const bf16_t* A, int lda, const bf16_t* 
 // rule puts the launch at (-1 where there is none).
 int gemm_ring_tile(int epi, bool rms, int M, int N, int K);
 long long gemm_ring_ns(int epi, bool rms, int M, int N, int K);
-// Columns of gemm_ring's EPI_CE tiles (of gemm()'s, 128, where the ring does
-// not fit): ceil(N / columns) partial sums per row.
-int gemm_ce_cols(const bf16_t* A, int lda, const bf16_t* W, int M, int N, int K,
-                 const EpiArgs& ea);
+// Columns of gemm_ring's EPI_CE tiles: ceil(N / columns) partial sums per row.
+int gemm_ce_cols(int M, int N, int K);
 // Dynamic LDS limits, once per device; called by the entry points before
 // anything they may capture into a graph.
 hipError_t gemm_ring_prepare();

@@ -8,7 +8,8 @@
 //  * k_gemm_sk / k_gemm_sk2: decode projections for 8 < M <= 128 rows on
 //    MFMA, one 16x16 or 32x32 output tile per work-group, K split over the
 //    four waves.
-//  * k_gemm / k_gemm_2w / k_gemm_bat: the lm_head's loss and top-k forms and
+//  * k_gemm / k_gemm_2w / k_gemm_bat: the lm_head's top-k form, its logits
+//    where the vocabulary is no multiple of 64, and
 //    batched products on MFMA (v_mfma_f32_16x16x32_bf16): 64..256 x 64..128 x
 //    64 tiles of four waves, swizzled LDS, register-prefetched K loop.  The
 //    other projections of the prefill are in gemm_ring.hip and gemm_big.hip.
@@ -542,9 +543,6 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   constexpr int WM = BM / 2, MT = WM / 16;   // rows per wave, 16-row MFMA tiles per wave
   constexpr int WN = BN / 2, NT = WN / 16;   // columns per wave, 16-column tiles per wave
   constexpr int CH = AC > BC ? AC : BC;
-  // the CE epilogue works on 128-column tiles (the per-tile partial sums of
-  // the loss)
-  static_assert(EPI != EPI_CE || BN == GM_BN, "128-column tiles");
   static_assert(EPI != EPI_TOPK || BN % 128 == 0, "whole 128-column candidate tiles");
   // staged epilogues (TOPK; PE_B / PE_X on full tiles) reuse the LDS for a bf16
   // BM x BN tile of row pitch BN + 8
@@ -720,49 +718,7 @@ __device__ __forceinline__ void gemm_body(const bf16_t* __restrict__ A, int lda,
   }
   // C^T layout: lane holds column m = (lane & 15) of its M block and rows
   // n = 4 (lane >> 4) + r, r = 0..3, of its N block
-  if constexpr (EPI == EPI_CE) {
-    // softcap(bf16(z)) in (0, 23): sum exp(zc) needs no max pass.  Row sums:
-    // in-lane over the wave's 4 N blocks, then over the 4 lane groups, then
-    // the two column halves (wn) through LDS, always in the same order.  The
-    // softcap and exp use the hardware exp2 / reciprocal: the IEEE expf and
-    // division cost ~35 VALU instructions per logit, over 1.65 G logits in the
-    // 64 x 512-token forward
-    float rs[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int m = m0 + wm * WM + i * 16 + r16;
-      const int tg = m < M ? ea.tgt[m] : -1;
-      float sum = 0.f;
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int n = n0 + wn * WN + j * 16 + (lane >> 4) * 4 + r;
-          if (n < N) {
-            const float zc = softcap_fast(bf2f(f2bf(acc[j][i][r])));
-            sum += __builtin_amdgcn_exp2f(zc * 1.4426950408889634f);
-            if (n == tg) ea.ce_tz[m] = zc;
-          }
-        }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      rs[i] = sum;
-    }
-    __syncthreads();   // LDS tiles no longer read: reuse for the halves
-    float* red = (float*)smem;
-    if (wn == 1 && lane < 16) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) red[wm * WM + i * 16 + r16] = rs[i];
-    }
-    __syncthreads();
-    if (wn == 0 && lane < 16) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = m0 + wm * WM + i * 16 + r16;
-        if (m < M) ea.ce_part[(size_t)tn * ea.ldz + m] = rs[i] + red[wm * WM + i * 16 + r16];
-      }
-    }
-  } else if constexpr (EPI == EPI_TOPK) {
+  if constexpr (EPI == EPI_TOPK) {
     __syncthreads();   // every wave is done with the last K tile in LDS
     constexpr int CP = BN + 8;
 #pragma unroll
@@ -1335,22 +1291,17 @@ hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N
   const int shape = M <= 64 ? 0 : M < 512 ? 1 : 2;
   const int bm = shape == 0 ? 64 : shape == 2 ? 256 : 128;
   dim3 grid((N + GM_BN - 1) / GM_BN, (M + bm - 1) / bm);
-#define ANN_GM_ONE(E, S)                                                                       \
-  if (S == 0)                                                                                  \
-    hipLaunchKernelGGL((k_gemm<E, 64, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K, ea); \
-  else if (S == 1)                                                                             \
-    hipLaunchKernelGGL((k_gemm<E, 128, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K,    \
-                       ea);                                                                    \
-  else                                                                                         \
-    hipLaunchKernelGGL((k_gemm_2w<E, 256, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M, N, K, \
-                       ea);
   switch (epi) {
     case EPI_LOGITS:
-      ANN_GM_ONE(EPI_LOGITS, shape)
-      break;
-    case EPI_CE:
-      if (!ea.ce_part || !ea.ce_tz || !ea.tgt || ea.ldz < M) return hipErrorInvalidValue;
-      ANN_GM_ONE(EPI_CE, shape)
+      if (shape == 0)
+        hipLaunchKernelGGL((k_gemm<EPI_LOGITS, 64, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M,
+                           N, K, ea);
+      else if (shape == 1)
+        hipLaunchKernelGGL((k_gemm<EPI_LOGITS, 128, GM_BN>), grid, dim3(256), 0, st, A, lda, W, M,
+                           N, K, ea);
+      else
+        hipLaunchKernelGGL((k_gemm_2w<EPI_LOGITS, 256, GM_BN>), grid, dim3(256), 0, st, A, lda, W,
+                           M, N, K, ea);
       break;
     case EPI_TOPK: {
       // decode rows only (the 64- and 128-row tiles); every 128 columns one record
@@ -1368,7 +1319,6 @@ hipError_t gemm(int epi, const bf16_t* A, int lda, const bf16_t* W, int M, int N
     default:
       return hipErrorInvalidValue;
   }
-#undef ANN_GM_ONE
   return hipGetLastError();
 }
 

@@ -44,10 +44,12 @@ def test_ring_gemm_logits_every_position(d, H, V, B, T):
     assert (got - R.logits(cfg, p, tok)).abs().max().item() < LOGIT_TOL
 
 
-# 128-column tiles, 192-column ones because nothing else divides the vocabulary
-# and because the rule prefers them; ragged last row blocks
-@pytest.mark.parametrize("d,H,V,B,T,cols", [(128, 1, 2432, 2, 150, 128), (128, 1, 2112, 2, 150, 192),
-                                            (192, 3, 2304, 5, 386, 192), (64, 1, 4608, 1, 33, 128)])
+# 128- and 192-column tiles, the last of them whole, of 64, 65 and 188 columns,
+# and the only one (70 columns); ragged last row blocks
+@pytest.mark.parametrize("d,H,V,B,T,cols", [(128, 1, 2432, 2, 150, 128), (128, 1, 2112, 2, 150, 128),
+                                            (128, 1, 2113, 2, 150, 128), (192, 3, 2304, 5, 386, 192),
+                                            (192, 3, 2300, 5, 386, 192), (64, 1, 4608, 1, 33, 128),
+                                            (64, 1, 70, 1, 20, 128)])
 def test_ring_gemm_loss_tiles(d, H, V, B, T, cols, traced):
     """Row losses and their mean; the suite's bounds of the training forward."""
     from attention_nn_amd.engine import Engine

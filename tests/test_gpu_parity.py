@@ -189,7 +189,7 @@ def test_prefill_wide_tiles(d, B, T):
 def test_forward_loss_matches_oracle(dh, V, B, T):
     """GPT.__call__ (model.py:180-221): per-row softcapped CE and the mean
     against the oracle's training forward (bf16 attention reading) and its
-    fp32 reading.  V = 1000 and 700 leave a partial last 128-column tile;
+    fp32 reading.  V = 1000 and 700 leave a partial last column tile;
     targets include 0 and V - 1."""
     cfg = GPTConfig(vocab_size=V, num_layers=2, num_heads=2, model_dim=2 * dh, seq_len=320,
                     window=70, long_layers=(1,))
@@ -212,8 +212,7 @@ def test_forward_loss_matches_oracle(dh, V, B, T):
 
 @pytest.mark.parametrize("V", [50304, 16384])
 def test_forward_loss_large_vocab_equals_cross_entropy_of_own_logits(V):
-    """The fused CE epilogue at the model's vocabulary (393 column tiles of 128,
-    the last partial) and at 1024 rows, against torch cross_entropy over the
+    """The fused CE epilogue at the model's vocabulary and at 1024 rows, against torch cross_entropy over the
     same engine's softcapped logits."""
     cfg = GPTConfig(vocab_size=V, num_layers=2, num_heads=2, model_dim=256, seq_len=512,
                     window=100, long_layers=(1,))
